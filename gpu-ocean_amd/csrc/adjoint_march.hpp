@@ -38,7 +38,10 @@ namespace adjm {
 constexpr int kLanes = 64;
 constexpr int kOut = 58;          // columns advanced per strip (lanes 3..60)
 
-using march::lane_get;
+// value of `v` in the lane whose byte address (lane * 4) is `addr`
+__device__ __forceinline__ float lane_get(float v, int addr) {
+    return __int_as_float(__builtin_amdgcn_ds_bpermute(addr, __float_as_int(v)));
+}
 
 // Launch arguments.  Planes of one array are `*_stride` bytes apart; the
 // record holds u, v, T, S and the code word in that order.

@@ -22,6 +22,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <stdint.h>
 
 namespace gocean {
@@ -31,9 +32,27 @@ constexpr float kDryEps = 1.0e-3f;     // CDKLM16_kernel.cu:38
 constexpr int kWall = 1;
 constexpr int kPeriodic = 2;
 
+// Constants derived from a domain's on the host, once per launch (or member
+// table) instead of in every thread; IEEE operations on either side, so the
+// same bits, and as kernel arguments or table entries they load into scalar
+// registers.
+struct SubstepDerived {
+    float vdx, udy, r_two_g, r_dx, r_dy;   // dx/(2g), dy/(2g), 1/(2g), 1/dx, 1/dy
+    float l_two_g, l_dx, l_dy;             // 1/d - RN(1/d), for div_k
+    float half_g, two_g, theta_g, dxf, dyf;   // 0.5 g, 2 g, theta g, dx f, dy f
+    // thresholds of the marching kernel's wave-uniform fast paths: a corner
+    // depth in (kDryFlag, plain_hi) is neither land nor the dry flag, and
+    // neither is the mean of four such; a face depth above face_lo is wet,
+    // needs no clamp at zero, and its wave speeds spread by at least
+    // flux_eps: with c = sqrt(g h), fl(max(u + c, 0)) - fl(min(u - c, 0)) >=
+    // 2 c (1 - 2^-22) for any u, so 2 sqrt(g h) (1 - 2^-20) >= flux_eps is
+    // enough
+    float plain_hi, face_lo;
+};
+
 // Everything one substep of one domain needs.  Plain launches pass it as a
 // kernel argument; the ensemble kernel builds it per workgroup from a table.
-struct SubstepArgs {
+struct SubstepArgs : SubstepDerived {
     const float* eta_in; const float* hu_in; const float* hv_in;
     const float* eta_qn; const float* hu_qn; const float* hv_qn;
     float* eta_out; float* hu_out; float* hv_out;
@@ -75,10 +94,6 @@ struct SubstepArgs {
     __host__ __device__ void set_rk_step(int step) {
         flags = (flags & ~(3u << 10)) | ((uint32_t)(step & 3) << 10);
     }
-    // derived by substep_derive on the host, once per launch instead of in
-    // every thread: dx/(2g), dy/(2g), 1/(2g), 1/dx, 1/dy (IEEE divisions on
-    // either side, so the same bits)
-    float vdx, udy, r_two_g, r_dx, r_dy;
     // branch record of the substep (written only by the recording variant):
     // per padded cell u, v, the x / y face depth terms and a code word
     float* tape_u; float* tape_v; float* tape_t; float* tape_s;
@@ -128,13 +143,30 @@ __device__ __forceinline__ void wind_grid_at(const float* grid, int wx, int wy, 
     Y = wind_lerp(wt, y0, y1);
 }
 
-inline void substep_derive(SubstepArgs& A) {
-    const float two_g = 2.0f * A.g;
-    A.vdx = A.dx / two_g;
-    A.udy = A.dy / two_g;
-    A.r_two_g = 1.0f / two_g;
-    A.r_dx = 1.0f / A.dx;
-    A.r_dy = 1.0f / A.dy;
+// 1/d - RN(1/d), rounded: the double quotient is off by 2^-53 relative, the
+// difference by about 2^-28 of itself
+inline float reciprocal_low(float d) { return (float)(1.0 / (double)d - (double)(1.0f / d)); }
+
+inline SubstepDerived substep_derive(float dx, float dy, float g, float theta, float f, float flux_eps, float cutoff,
+                                     float land) {
+    SubstepDerived D;
+    D.half_g = 0.5f * g;
+    D.two_g = 2.0f * g;
+    D.theta_g = theta * g;
+    D.dxf = dx * f;
+    D.dyf = dy * f;
+    D.vdx = dx / D.two_g;
+    D.udy = dy / D.two_g;
+    D.r_two_g = 1.0f / D.two_g;
+    D.r_dx = 1.0f / dx;
+    D.r_dy = 1.0f / dy;
+    D.l_two_g = reciprocal_low(D.two_g);
+    D.l_dx = reciprocal_low(dx);
+    D.l_dy = reciprocal_low(dy);
+    D.plain_hi = (land >= 1.0f) ? 0.5f * land : -INFINITY;
+    const float c = 0.50001f * flux_eps;
+    D.face_lo = fmaxf(fmaxf(cutoff, 0.0f), (c * c) / g * 1.00001f);
+    return D;
 }
 
 // ---------------------------------------------------------------------------
@@ -150,6 +182,13 @@ __host__ __device__ __forceinline__ float minmod_raw(float b, float c, float f) 
     const uint32_t uf = __builtin_bit_cast(uint32_t, f);
     const bool agree = (((ub ^ uc) | (uc ^ uf)) & 0x80000000u) == 0u;
     return agree ? copysignf(m, b) : 0.0f;
+}
+
+// The same as a median: the least of three positive candidates, the greatest
+// of three negative ones, zero between them.  Three instructions (min3, max3,
+// med3) against five; the value is minmod_raw's, up to the sign of a zero.
+__device__ __forceinline__ float minmod3(float b, float c, float f) {
+    return __builtin_amdgcn_fmed3f(fminf(fminf(b, c), f), fmaxf(fmaxf(b, c), f), 0.0f);
 }
 
 // common.cu:532-542
@@ -217,21 +256,17 @@ __device__ __forceinline__ float div_r(float n, float d, float r) {
     return fmaf(e, r, q);
 }
 
-// n/d for a launch-constant divisor d (dx, dy, 2g) with r = RN(1/d) formed on
-// the host: one residual correction.  The host enables it (SubstepArgs
-// fast_arith()) only for divisors for which it has checked, over every float
-// significand of n, that this gives the correctly rounded quotient (see
-// fast_arith_exact in gocean_fwd.hip); otherwise div_r's two corrections are
-// used.
-__device__ __forceinline__ float div_c1(float n, float d, float r) {
-    const float q = n * r;
-    const float e = fmaf(-d, q, n);
-    return fmaf(e, r, q);
-}
-
+// n/d for a launch-constant divisor d (dx, dy, 2g): with the reciprocal as an
+// unevaluated sum r + l (r = RN(1/d), l = RN(1/d - r), formed on the host),
+// RN(n r + RN(n l)) in two instructions (Brisebarre, Muller & Raina,
+// "Accelerating correctly rounded floating-point division when the divisor is
+// known in advance", IEEE Trans. Computers 53 (2004); div_r takes five).  It
+// is correctly rounded for most divisors; the host enables it (SubstepArgs
+// fast_arith()) only for divisors for which it has checked every float
+// significand of n (fast_arith_exact in gocean_fwd.hip); otherwise div_r runs.
 template <bool FAST>
-__device__ __forceinline__ float div_k(float n, float d, float r) {
-    if constexpr (FAST) return div_c1(n, d, r);
+__device__ __forceinline__ float div_k(float n, float d, float r, float l) {
+    if constexpr (FAST) return fmaf(n, r, n * l);
     else return div_r(n, d, r);
 }
 
@@ -270,11 +305,9 @@ __device__ __forceinline__ float sqrt_k(float x) {
     else return sqrt_rn(x);
 }
 
-struct Consts {
-    float g, half_g, two_g, theta, theta_g;
-    float dx, dy, vdx, udy;        // vdx = DX/(2g), udy = DY/(2g)
+struct Consts : SubstepDerived {
+    float g, theta, dx, dy;
     float desing, flux_eps, cutoff, land;
-    float r_two_g, r_dx, r_dy;     // RN(1/(2g)), RN(1/dx), RN(1/dy)
 };
 
 // Central-upwind flux of primitive face states Qm=(hm,um,vm), Qp=(hp,up,vp)
@@ -375,22 +408,15 @@ __device__ __forceinline__ int xcd_band(int b, int nb) {
 
 __device__ __forceinline__ Consts make_consts(const SubstepArgs& A) {
     Consts K;
+    static_cast<SubstepDerived&>(K) = A;
     K.g = A.g;
-    K.half_g = 0.5f * A.g;
-    K.two_g = 2.0f * A.g;
     K.theta = A.theta;
-    K.theta_g = A.theta * A.g;
     K.dx = A.dx;
     K.dy = A.dy;
-    K.vdx = A.vdx;
-    K.udy = A.udy;
     K.desing = A.desing_eps;
     K.flux_eps = A.flux_eps;
     K.cutoff = A.cutoff;
     K.land = A.land;
-    K.r_two_g = A.r_two_g;
-    K.r_dx = A.r_dx;
-    K.r_dy = A.r_dy;
     return K;
 }
 

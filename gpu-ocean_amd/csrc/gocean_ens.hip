@@ -23,7 +23,7 @@
 namespace gocean {
 
 // one member as the device sees it
-struct EnsMember {
+struct EnsMember : SubstepDerived {
     int nx, ny, pitch, hi_pitch;
     long long state_off, plane, hi_off, hm_off, field_off;
     int tiles_x, tile_begin;
@@ -31,14 +31,13 @@ struct EnsMember {
     float f, north_x, north_y;
     float wind_x, wind_y;          // wind stress (wind_lerp of the member's samples)
     int bc_n, bc_e, bc_s, bc_w;
-    float vdx, udy;                // as SubstepArgs (with r_dx, r_dy, r_two_g below)
     // reverse mode (set by gocean_ensemble_adjoint_setup): the member's block
     // of the work buffer and its tiles in the recording-forward (32x16) and
     // adjoint (kAdjBW x kAdjBH) launches
     long long work_off;
     int ftiles_x, ftile_begin, atiles_x, atile_begin;
     int astrips_x, astrip_begin;   // the member's strips in the column-marching reverse launch
-    float r_dx, r_dy, r_two_g, Dx, Dy, Ddx, Ddy, g_dx, g_dy;   // as AdjTileArgs / SubstepArgs
+    float Dx, Dy, Ddx, Ddy, g_dx, g_dy;   // as AdjTileArgs
 };
 
 struct EnsLaunch {
@@ -80,14 +79,14 @@ __device__ __forceinline__ void member_args(const EnsLaunch& L, const EnsMember&
     A.wind_grid = nullptr; A.wind_wx = 0; A.wind_wy = 0; A.wind_t = 0.0f;   // members: uniform wind
     A.dt = 0.0f;
     A.set_flags(M.bc_n, M.bc_e, M.bc_s, M.bc_w, L.rk_order, L.rk_step);
-    A.vdx = M.vdx; A.udy = M.udy; A.r_two_g = M.r_two_g; A.r_dx = M.r_dx; A.r_dy = M.r_dy;
+    static_cast<SubstepDerived&>(A) = M;
     A.tiles_x = M.tiles_x; A.tiles_y = 0;
 }
 
 // column-marching substep over every member's strips: wavefront -> strip
 // through the tile map (one entry per strip), as k_march
-template <bool FAST>
-__global__ __launch_bounds__(256) void k_ens_march(EnsLaunch L) {
+template <bool FAST, int STAGE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_ens_march(EnsLaunch L) {
     const int wave = xcd_band(blockIdx.x, gridDim.x) * 4 + march::wave_in_group();
     if (wave >= L.n_tiles) return;
     const int m = L.tile_member[wave];
@@ -97,7 +96,7 @@ __global__ __launch_bounds__(256) void k_ens_march(EnsLaunch L) {
     member_args<kModeZero>(L, M, m, A);
     const int lt = wave - M.tile_begin;
     const int sy = lt / M.tiles_x, sx = lt - sy * M.tiles_x;
-    march::march_strip<FAST, false>(A, sx, sy, L.march_bh);   // members: uniform wind
+    march::march_strip<FAST, false, STAGE>(A, sx, sy, L.march_bh);   // members: uniform wind
 }
 
 template <int BW, int BH, int NT, int MODE>
@@ -287,7 +286,7 @@ __global__ __launch_bounds__(kEnsTapeNT) __attribute__((amdgpu_waves_per_eu(8)))
     A.wind_grid = nullptr; A.wind_wx = 0; A.wind_wy = 0; A.wind_t = 0.0f;   // members: uniform wind
     A.dt = 0.0f;
     A.set_flags(M.bc_n, M.bc_e, M.bc_s, M.bc_w, 2, L.rk_step);
-    A.vdx = M.vdx; A.udy = M.udy; A.r_two_g = M.r_two_g; A.r_dx = M.r_dx; A.r_dy = M.r_dy;
+    static_cast<SubstepDerived&>(A) = M;
     A.tiles_x = M.ftiles_x; A.tiles_y = 0;
     const int lt = t - M.ftile_begin;
     const int ty = lt / M.ftiles_x, tx = lt - ty * M.ftiles_x;
@@ -327,11 +326,11 @@ __global__ __launch_bounds__(256) void k_ens_march_tape(EnsTapeLaunch L, int bh,
     A.wind_grid = nullptr; A.wind_wx = 0; A.wind_wy = 0; A.wind_t = 0.0f;   // members: uniform wind
     A.dt = 0.0f;
     A.set_flags(M.bc_n, M.bc_e, M.bc_s, M.bc_w, 2, L.rk_step);
-    A.vdx = M.vdx; A.udy = M.udy; A.r_two_g = M.r_two_g; A.r_dx = M.r_dx; A.r_dy = M.r_dy;
+    static_cast<SubstepDerived&>(A) = M;
     A.tiles_x = M.tiles_x; A.tiles_y = 0;
     const int lt = wave - M.tile_begin;
     const int sy = lt / M.tiles_x, sx = lt - sy * M.tiles_x;
-    march::march_strip<FAST, false, true>(A, sx, sy, bh);
+    march::march_strip<FAST, false, march::kStageAny, true>(A, sx, sy, bh);
 }
 
 struct EnsAdjLaunch {
@@ -458,6 +457,7 @@ struct gocean_ensemble {
     int n_tiles = 0;
     int device = 0;
     bool fast_arith = false;   // fast_arith_exact holds for every member
+    float friction = 0.0f;     // largest r of the members
     EnsMember* d_members = nullptr;
     int* d_tile_member = nullptr;
     std::vector<EnsMember> members;
@@ -485,12 +485,20 @@ static void ens_launch_t(const EnsLaunch& L, hipStream_t s) {
     hipLaunchKernelGGL((k_ens_substep<BW, BH, NT, MODE>), dim3(L.n_tiles), dim3(NT), 0, s, L);
 }
 
-static void ens_march(EnsLaunch L, int bh, bool fast_arith, hipStream_t s) {
+using EnsKernel = void (*)(EnsLaunch);
+template <bool FAST>
+static EnsKernel ens_march_kernel(int stage) {
+    return stage == march::kStageFirst ? k_ens_march<FAST, march::kStageFirst>
+         : stage == march::kStageSecond ? k_ens_march<FAST, march::kStageSecond>
+                                        : k_ens_march<FAST, march::kStageAny>;
+}
+
+// r: the largest friction coefficient of the members
+static void ens_march(EnsLaunch L, int bh, bool fast_arith, float r, hipStream_t s) {
     L.march_bh = bh;
-    if (fast_arith)
-        hipLaunchKernelGGL((k_ens_march<true>), dim3((L.n_tiles + 3) / 4), dim3(256), 0, s, L);
-    else
-        hipLaunchKernelGGL((k_ens_march<false>), dim3((L.n_tiles + 3) / 4), dim3(256), 0, s, L);
+    const int stage = march_stage(L.rk_order, L.rk_step, r);
+    hipLaunchKernelGGL(fast_arith ? ens_march_kernel<true>(stage) : ens_march_kernel<false>(stage),
+                       dim3((L.n_tiles + 3) / 4), dim3(256), 0, s, L);
 }
 
 // rows per strip of the ensemble's column-marching launch (configuration
@@ -501,7 +509,9 @@ static int ens_march_rows(const std::vector<EnsMember>& members, bool fast_arith
         strips.push_back((M.nx + march::kOut - 1) / march::kOut);
         ny.push_back(M.ny);
     }
-    const int resident = resident_waves(fast_arith ? (const void*)k_ens_march<true> : (const void*)k_ens_march<false>);
+    // the second stage is the larger kernel of the two
+    const int resident = resident_waves((const void*)(fast_arith ? ens_march_kernel<true>(march::kStageSecond)
+                                                                 : ens_march_kernel<false>(march::kStageSecond)));
     return march_rows(strips.data(), ny.data(), (int)members.size(), resident);
 }
 
@@ -524,7 +534,7 @@ static int ens_launch(const gocean_ensemble* E, EnsLaunch L, hipStream_t s) {
             case 6: ens_launch_t<32, 14, 512, kModeZero>(L, s); break;
             case 7:
             case 8:
-            case 9: ens_march(L, E->bh, E->fast_arith, s); break;
+            case 9: ens_march(L, E->bh, E->fast_arith, E->friction, s); break;
         }
     }
     return check_launch("ensemble substep launch");
@@ -612,9 +622,11 @@ int gocean_ensemble_create(const gocean_member_t* members, int n, int tile_confi
         E->cfg = kDefaultTileConfig;
     }
     E->fast_arith = true;
+    E->friction = 0.0f;
     for (int k = 0; k < n; ++k) {
         const gocean_domain_t& d = members[k].domain;
         E->fast_arith = E->fast_arith && fast_arith_exact(d.g, d.dx, d.dy, d.depth_cutoff);
+        E->friction = std::max(E->friction, d.r);
     }
     const TileConfig& tc = (E->mode == kModeZero) ? kTileConfigs[E->cfg] : kTileConfigs[0];
     E->bw = tc.bw; E->bh = tc.bh; E->nt = tc.nt;
@@ -647,13 +659,8 @@ int gocean_ensemble_create(const gocean_member_t* members, int n, int tile_confi
         M.wind_x = wind_lerp(m.wind.t, m.wind.x0, m.wind.x1);
         M.wind_y = wind_lerp(m.wind.t, m.wind.y0, m.wind.y1);
         M.bc_n = d.bc_north; M.bc_e = d.bc_east; M.bc_s = d.bc_south; M.bc_w = d.bc_west;
-        {
-            SubstepArgs D;
-            std::memset(&D, 0, sizeof(D));
-            D.dx = d.dx; D.dy = d.dy; D.g = d.g;
-            substep_derive(D);
-            M.vdx = D.vdx; M.udy = D.udy; M.r_two_g = D.r_two_g; M.r_dx = D.r_dx; M.r_dy = D.r_dy;
-        }
+        static_cast<SubstepDerived&>(M) =
+            substep_derive(d.dx, d.dy, d.g, d.theta, d.f, d.flux_slope_eps, d.depth_cutoff, d.land_value);
         if (m.state_offset < 0 || m.hi_offset < 0 || m.hm_offset < 0) {
             delete E;
             return set_error(GOCEAN_EINVAL, "member %d: negative buffer offset", k);

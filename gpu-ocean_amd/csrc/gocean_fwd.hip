@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -72,40 +73,34 @@ int validate_domain(const gocean_domain_t* d) {
 }
 
 // ---------------------------------------------------------------------------
-// division by a launch constant with one residual correction
+// division by a launch constant in two instructions
 // ---------------------------------------------------------------------------
-// For q = RN(n r), r = RN(1/d), one correction RN(q + RN(n - d q) r) is the
-// correctly rounded n/d for most d but is not guaranteed for all.  Scaling n
-// by a power of two scales q, the residual and the quotient exactly, so the
-// check over the 2^23 significands of n in [1, 2) decides it for every n of
-// normal magnitude (and -n by symmetry).  Done once per divisor value on the
-// host, with the hardware FMA when the CPU has one.
+// RN(n r + RN(n l)) with r = RN(1/d), l = RN(1/d - r) (div_k) is the correctly
+// rounded n/d for most d but is not guaranteed for all.  Scaling n by a power
+// of two scales every intermediate exactly, so the check over the 2^23
+// significands of n in [1, 2) decides it for every n of normal magnitude (and
+// -n by symmetry).  Done once per divisor value on the host, with the hardware
+// FMA when the CPU has one.
 namespace {
 
-__attribute__((target("fma"))) bool one_correction_scan_fma(float d) {
-    const float r = 1.0f / d;
+__attribute__((target("fma"))) bool two_step_scan_fma(float d) {
+    const float r = 1.0f / d, l = reciprocal_low(d);
     for (uint32_t m = 0; m < (1u << 23); ++m) {
         uint32_t bits = 0x3f800000u | m;
         float n;
         std::memcpy(&n, &bits, 4);
-        const float q = n * r;
-        const float e = __builtin_fmaf(-d, q, n);
-        const float q1 = __builtin_fmaf(e, r, q);
-        if (q1 != n / d) return false;
+        if (__builtin_fmaf(n, r, n * l) != n / d) return false;
     }
     return true;
 }
 
-bool one_correction_scan_libm(float d) {
-    const float r = 1.0f / d;
+bool two_step_scan_libm(float d) {
+    const float r = 1.0f / d, l = reciprocal_low(d);
     for (uint32_t m = 0; m < (1u << 23); ++m) {
         uint32_t bits = 0x3f800000u | m;
         float n;
         std::memcpy(&n, &bits, 4);
-        const float q = n * r;
-        const float e = std::fmaf(-d, q, n);
-        const float q1 = std::fmaf(e, r, q);
-        if (q1 != n / d) return false;
+        if (std::fmaf(n, r, n * l) != n / d) return false;
     }
     return true;
 }
@@ -115,7 +110,7 @@ std::unordered_map<uint32_t, bool> g_div_ok;
 
 }  // namespace
 
-bool one_correction_exact(float d) {
+bool two_step_exact(float d) {
     if (!(d > 0.0f) || !std::isnormal(d) || !std::isnormal(1.0f / d)) return false;
     uint32_t key;
     std::memcpy(&key, &d, 4);
@@ -124,7 +119,7 @@ bool one_correction_exact(float d) {
         auto it = g_div_ok.find(key);
         if (it != g_div_ok.end()) return it->second;
     }
-    const bool ok = __builtin_cpu_supports("fma") ? one_correction_scan_fma(d) : one_correction_scan_libm(d);
+    const bool ok = __builtin_cpu_supports("fma") ? two_step_scan_fma(d) : two_step_scan_libm(d);
     std::lock_guard<std::mutex> lock(g_div_mu);
     g_div_ok[key] = ok;
     return ok;
@@ -135,7 +130,7 @@ bool fast_arith_exact(float g, float dx, float dy, float cutoff) {
     // it only for depths above the cutoff, whose g h rounds to >= RN(g cutoff)
     const float lo = g * cutoff;
     if (!(g > 0.0f) || !std::isfinite(g) || !(lo >= 0x1p-60f)) return false;
-    return one_correction_exact(2.0f * g) && one_correction_exact(dx) && one_correction_exact(dy);
+    return two_step_exact(2.0f * g) && two_step_exact(dx) && two_step_exact(dy);
 }
 
 void fill_args(const gocean_domain_t* d, SubstepArgs& A) {
@@ -146,7 +141,8 @@ void fill_args(const gocean_domain_t* d, SubstepArgs& A) {
     A.cutoff = d->depth_cutoff; A.land = d->land_value;
     A.f = d->f; A.north_x = d->north_x; A.north_y = d->north_y;
     A.set_flags(d->bc_north, d->bc_east, d->bc_south, d->bc_west, d->rk_order, 0);
-    substep_derive(A);
+    static_cast<SubstepDerived&>(A) =
+        substep_derive(A.dx, A.dy, A.g, A.theta, A.f, A.flux_eps, A.cutoff, A.land);
     A.set_fast_arith(fast_arith_exact(A.g, A.dx, A.dy, A.cutoff));
 }
 
@@ -189,12 +185,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 512 ? 
 
 // column-marching substep: wavefront w of the grid takes strip (sx, sy),
 // sx fastest, workgroups banded over the XCDs
-template <bool FAST, bool WGRID>
-__global__ __launch_bounds__(256) void k_march(SubstepArgs A) {
+template <bool FAST, bool WGRID, int STAGE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WGRID ? 4 : 5))) void k_march(SubstepArgs A) {
     const int wave = xcd_band(blockIdx.x, gridDim.x) * 4 + march::wave_in_group();
     if (wave >= A.tiles_x * A.tiles_y) return;
     const int sy = wave / A.tiles_x, sx = wave - sy * A.tiles_x;
-    march::march_strip<FAST, WGRID>(A, sx, sy, A.march_bh);
+    march::march_strip<FAST, WGRID, STAGE>(A, sx, sy, A.march_bh);
 }
 
 // waves of a kernel that the device holds at once: 4 SIMDs per CU, each
@@ -231,10 +227,23 @@ int march_rows(const int* strips, const int* ny, int n, int resident) {
     return best;
 }
 
-// the marching kernel for the launch's arithmetic and wind variants
-static const void* march_kernel(bool fast, bool wgrid) {
-    if (fast) return wgrid ? (const void*)k_march<true, true> : (const void*)k_march<true, false>;
-    return wgrid ? (const void*)k_march<false, true> : (const void*)k_march<false, false>;
+// the marching kernel of the launch's arithmetic, wind and stage
+using SubstepKernel = void (*)(SubstepArgs);
+template <bool FAST, bool WGRID>
+static SubstepKernel march_kernel_of(int stage) {
+    return stage == march::kStageFirst ? k_march<FAST, WGRID, march::kStageFirst>
+         : stage == march::kStageSecond ? k_march<FAST, WGRID, march::kStageSecond>
+                                        : k_march<FAST, WGRID, march::kStageAny>;
+}
+static SubstepKernel march_kernel(bool fast, bool wgrid, int stage) {
+    if (fast) return wgrid ? march_kernel_of<true, true>(stage) : march_kernel_of<true, false>(stage);
+    return wgrid ? march_kernel_of<false, true>(stage) : march_kernel_of<false, false>(stage);
+}
+
+// the stage instantiation of a substep
+int march_stage(int rk_order, int rk_step, float r) {
+    if (rk_order > 2 || r > 0.0f) return march::kStageAny;
+    return rk_step == 0 ? march::kStageFirst : march::kStageSecond;
 }
 
 // sqrt_newton against sqrt_rn over the float bit patterns lo .. hi
@@ -253,23 +262,18 @@ __global__ __launch_bounds__(256) void k_sqrt_check(uint32_t lo, uint32_t hi, un
 static void launch_march(SubstepArgs A, int bh, hipStream_t s) {
     A.tiles_x = (A.nx + march::kOut - 1) / march::kOut;
     const bool fast = A.fast_arith(), wgrid = A.wind_grid != nullptr;
+    const int stage = march_stage(A.rk_order(), A.rk_step(), A.r);
+    const SubstepKernel kernel = march_kernel(fast, wgrid, stage);
     if (bh <= 0) {
-        static int resident[4] = {0, 0, 0, 0};
-        const int k = (fast ? 2 : 0) + (wgrid ? 1 : 0);
-        if (!resident[k]) resident[k] = resident_waves(march_kernel(fast, wgrid));
-        bh = march_rows(&A.tiles_x, &A.ny, 1, resident[k]);
+        static std::atomic<int> resident[12];
+        std::atomic<int>& res = resident[(fast ? 6 : 0) + (wgrid ? 3 : 0) + stage];
+        if (!res.load()) res.store(resident_waves((const void*)kernel));
+        bh = march_rows(&A.tiles_x, &A.ny, 1, res.load());
     }
     A.march_bh = bh;
     A.tiles_y = (A.ny + bh - 1) / bh;
     const int waves = A.tiles_x * A.tiles_y;
-    const dim3 grid((waves + 3) / 4), block(256);
-    if (fast) {
-        if (wgrid) hipLaunchKernelGGL((k_march<true, true>), grid, block, 0, s, A);
-        else hipLaunchKernelGGL((k_march<true, false>), grid, block, 0, s, A);
-    } else {
-        if (wgrid) hipLaunchKernelGGL((k_march<false, true>), grid, block, 0, s, A);
-        else hipLaunchKernelGGL((k_march<false, false>), grid, block, 0, s, A);
-    }
+    hipLaunchKernelGGL(kernel, dim3((waves + 3) / 4), dim3(256), 0, s, A);
 }
 
 template <int BW, int BH, int NT, int MODE>
@@ -305,7 +309,7 @@ __global__ __launch_bounds__(256) void k_march_tape(SubstepArgs A) {
     const int wave = xcd_band(blockIdx.x, gridDim.x) * 4 + march::wave_in_group();
     if (wave >= A.tiles_x * A.tiles_y) return;
     const int sy = wave / A.tiles_x, sx = wave - sy * A.tiles_x;
-    march::march_strip<FAST, false, true>(A, sx, sy, A.march_bh);
+    march::march_strip<FAST, false, march::kStageAny, true>(A, sx, sy, A.march_bh);
 }
 
 // bh > 0: fixed rows per strip; 0: balanced by march_rows

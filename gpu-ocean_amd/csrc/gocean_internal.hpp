@@ -32,7 +32,7 @@ int validate_domain(const gocean_domain_t* d);
 void fill_args(const gocean_domain_t* d, SubstepArgs& A);
 // true when one residual correction divides every float by d correctly
 // rounded (checked once per value of d, on the host)
-bool one_correction_exact(float d);
+bool two_step_exact(float d);
 // the substep's FAST arithmetic is exact for these constants: one-correction
 // division by dx, dy and 2g, and the Newton square root of g h for h above
 // the depth cutoff
@@ -43,6 +43,7 @@ bool march_fits(int ny, int pitch, int hi_pitch);
 // column-marching launch shape: waves the device holds at once for a kernel,
 // and the rows per strip that fill whole rounds of them
 int resident_waves(const void* kernel);
+int march_stage(int rk_order, int rk_step, float r);
 int march_rows(const int* strips, const int* ny, int n, int resident);
 int launch_substep(const SubstepArgs& A, int cfg, bool field, hipStream_t s);
 // zero-rotation substep that also writes the branch record (A.tape_*)
