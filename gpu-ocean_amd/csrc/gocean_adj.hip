@@ -54,7 +54,7 @@ int adj_march_rows(const int* nx, const int* ny, int n) {
         strips[k] = (nx[k] + adjm::kOut - 1) / adjm::kOut;
         rows[k] = ny[k] + 4;
     }
-    return march_rows(strips.data(), rows.data(), n, resident);
+    return march_rows(strips.data(), rows.data(), n, resident, 8);
 }
 
 __global__ __launch_bounds__(256) void k_adj_fold(FoldArgs F) {

@@ -458,6 +458,7 @@ struct gocean_ensemble {
     int device = 0;
     bool fast_arith = false;   // fast_arith_exact holds for every member
     float friction = 0.0f;     // largest r of the members
+    bool fits = true;          // every member's planes suit the marching kernel's 32-bit offsets
     EnsMember* d_members = nullptr;
     int* d_tile_member = nullptr;
     std::vector<EnsMember> members;
@@ -512,7 +513,7 @@ static int ens_march_rows(const std::vector<EnsMember>& members, bool fast_arith
     // the second stage is the larger kernel of the two
     const int resident = resident_waves((const void*)(fast_arith ? ens_march_kernel<true>(march::kStageSecond)
                                                                  : ens_march_kernel<false>(march::kStageSecond)));
-    return march_rows(strips.data(), ny.data(), (int)members.size(), resident);
+    return march_rows(strips.data(), ny.data(), (int)members.size(), resident, 1);
 }
 
 static int ens_launch(const gocean_ensemble* E, EnsLaunch L, hipStream_t s) {
@@ -584,10 +585,7 @@ int gocean_ensemble_create(const gocean_member_t* members, int n, int tile_confi
     if (!E) return set_error(GOCEAN_ENOMEM, "host allocation failed");
     E->n = n;
     E->rk_order = members[0].domain.rk_order;
-    long long mean_cells = 0;
-    for (int k = 0; k < n; ++k) mean_cells += (long long)members[k].domain.nx * members[k].domain.ny;
-    mean_cells /= n;
-    E->cfg = tile_config < 0 ? default_tile_config(mean_cells) : tile_config;
+    E->cfg = tile_config < 0 ? default_tile_config() : tile_config;
     bool any_field = false, any_const = false;
     for (int k = 0; k < n; ++k) {
         const gocean_domain_t& d = members[k].domain;
@@ -610,10 +608,9 @@ int gocean_ensemble_create(const gocean_member_t* members, int n, int tile_confi
             }
     }
     E->mode = any_field ? kModeField : (any_const ? kModeConst : kModeZero);
-    bool fits = true;
     for (int k = 0; k < n; ++k)
-        fits = fits && march_fits(members[k].domain.ny, members[k].domain.pitch, members[k].domain.hi_pitch);
-    if (E->cfg >= kFirstMarchConfig && !fits) {
+        E->fits = E->fits && march_fits(members[k].domain.ny, members[k].domain.pitch, members[k].domain.hi_pitch);
+    if (E->cfg >= kFirstMarchConfig && !E->fits) {
         if (tile_config >= 0) {
             delete E;
             return set_error(GOCEAN_EINVAL, "tile configuration %d (column marching) needs member planes below 4 GiB",
@@ -691,13 +688,12 @@ int gocean_ensemble_create(const gocean_member_t* members, int n, int tile_confi
 int gocean_ensemble_set_tile_config(gocean_ensemble_t* E, int tile_config) {
     clear_error();
     if (!E) return set_error(GOCEAN_EINVAL, "ensemble is NULL");
-    if (tile_config < 0) {
-        long long mean_cells = 0;
-        for (const EnsMember& M : E->members) mean_cells += (long long)M.nx * M.ny;
-        tile_config = default_tile_config(mean_cells / E->n);
-    }
     if (tile_config >= kNumTileConfigs)
         return set_error(GOCEAN_EINVAL, "tile configuration %d out of range", tile_config);
+    if (tile_config >= kFirstMarchConfig && !E->fits)
+        return set_error(GOCEAN_EINVAL, "tile configuration %d (column marching) needs member planes below 4 GiB",
+                         tile_config);
+    if (tile_config < 0) tile_config = E->fits ? default_tile_config() : kDefaultTileConfig;
     // work already queued may still read the old tables
     if (hipDeviceSynchronize() != hipSuccess) return check_launch("ensemble tile configuration");
     E->cfg = tile_config;
@@ -891,7 +887,7 @@ long long gocean_ensemble_adjoint_setup(gocean_ensemble_t* E, int max_steps) {
     }
     static int resident = 0;
     if (!resident) resident = resident_waves((const void*)k_ens_adj_march);
-    const int abh = march_rows(snx.data(), sny.data(), E->n, resident);
+    const int abh = march_rows(snx.data(), sny.data(), E->n, resident, 8);
     for (int k = 0; k < E->n; ++k) {
         EnsMember& M = E->members[k];
         M.astrips_x = snx[k];

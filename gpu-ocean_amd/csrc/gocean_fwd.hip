@@ -210,14 +210,17 @@ int resident_waves(const void* kernel) {
     return cus * 4 * per_simd;
 }
 
-// Rows per strip for the column-marching kernel over domains of the given
+// Rows per strip for a column-marching kernel over domains of the given
 // strip counts and heights: each wave's time grows with its rows plus about
 // three rows of prologue, and waves run in rounds of `resident`; pick the
-// row count (8..256) with the least rounds * (rows + 3).
-int march_rows(const int* strips, const int* ny, int n, int resident) {
-    int best = 8;
+// row count (least..256) with the least rounds * (rows + 3).  Measured over
+// fixed row counts, the choice is the best or within 3 % of it from 96x80 (1
+// row) over 512^2 (1), 1024^2 (4) and 2048^2 (15) to 1024 members of 64^2 and
+// 100 of 512^2.
+int march_rows(const int* strips, const int* ny, int n, int resident, int least) {
+    int best = least;
     double best_cost = 1e300;
-    for (int bh = 8; bh <= 256; ++bh) {
+    for (int bh = least; bh <= 256; ++bh) {
         long long waves = 0;
         for (int k = 0; k < n; ++k) waves += (long long)strips[k] * ((ny[k] + bh - 1) / bh);
         const long long rounds = (waves + resident - 1) / resident;
@@ -225,6 +228,20 @@ int march_rows(const int* strips, const int* ny, int n, int resident) {
         if (cost < best_cost - 1e-9) { best_cost = cost; best = bh; }
     }
     return best;
+}
+
+// march_rows of one domain.  The search takes microseconds, as long as a
+// launch, so each thread keeps its last answers by value.
+static int march_rows_one(int strips, int ny, int resident) {
+    struct Entry { int strips, ny, resident, rows; };
+    static thread_local Entry memo[4] = {};
+    static thread_local int next = 0;
+    for (const Entry& e : memo)
+        if (e.strips == strips && e.ny == ny && e.resident == resident) return e.rows;
+    const int rows = march_rows(&strips, &ny, 1, resident, 1);
+    memo[next] = Entry{strips, ny, resident, rows};
+    next = (next + 1) & 3;
+    return rows;
 }
 
 // the marching kernel of the launch's arithmetic, wind and stage
@@ -268,7 +285,7 @@ static void launch_march(SubstepArgs A, int bh, hipStream_t s) {
         static std::atomic<int> resident[12];
         std::atomic<int>& res = resident[(fast ? 6 : 0) + (wgrid ? 3 : 0) + stage];
         if (!res.load()) res.store(resident_waves((const void*)kernel));
-        bh = march_rows(&A.tiles_x, &A.ny, 1, res.load());
+        bh = march_rows_one(A.tiles_x, A.ny, res.load());
     }
     A.march_bh = bh;
     A.tiles_y = (A.ny + bh - 1) / bh;
@@ -320,7 +337,7 @@ static void launch_march_tape(SubstepArgs A, int bh, hipStream_t s) {
         static int resident[2] = {0, 0};
         const void* k = fast ? (const void*)k_march_tape<true> : (const void*)k_march_tape<false>;
         if (!resident[fast]) resident[fast] = resident_waves(k);
-        bh = march_rows(&A.tiles_x, &A.ny, 1, resident[fast]);
+        bh = march_rows_one(A.tiles_x, A.ny, resident[fast]);
     }
     A.march_bh = bh;
     A.tiles_y = (A.ny + bh - 1) / bh;
@@ -330,13 +347,14 @@ static void launch_march_tape(SubstepArgs A, int bh, hipStream_t s) {
 }
 
 // tile configuration of the recording forward (process-wide; the record is
-// laid out per cell, so every configuration writes the same record); -1:
-// the column-marching kernel from a million cells on, 32x16/512 below
+// laid out per cell, so every configuration writes the same record); -1: the
+// column-marching kernel (per substep against 32x16/512: 96^2 8.4 / 11.3 us,
+// 512^2 13.7 / 15.1, 1024^2 25.2 / 36.0)
 static int g_record_cfg = -1;
 
 int launch_substep_tape(SubstepArgs A, hipStream_t s) {
     int cfg = g_record_cfg;
-    if (cfg < 0) cfg = default_tile_config((long long)A.nx * A.ny) >= kFirstMarchConfig ? kMarchAutoConfig : 5;
+    if (cfg < 0) cfg = kMarchAutoConfig;
     if (cfg >= kFirstMarchConfig && !march_fits(A.ny, A.pitch, A.hi_pitch)) cfg = 5;
     switch (cfg) {
         case 0: launch_tape_t<32, 8, 256>(A, s); break;
@@ -358,9 +376,13 @@ int substep_mode(const SubstepArgs& A, bool field) {
     return (A.north_x == 0.0f && A.north_y == 1.0f) ? kModeZero : kModeConst;
 }
 
-// default configuration: the column-marching kernel with balanced rows
-// per strip from a million cells on (where it is faster), else the 2-D tile
-int default_tile_config(long long cells) { return cells >= (1LL << 20) ? kMarchAutoConfig : kDefaultTileConfig; }
+// Default configuration: the column-marching kernel with balanced rows per
+// strip, for every size.  Small domains get strips of few rows (march_rows),
+// so that they too spread over the chip.  Substep times, marching against the
+// best 2-D tile: 96x80 5.5 / 7.5 us, 512^2 8.5 / 9.1, 1024^2 16.4 / 23.7,
+// 2048^2 43.8 / 74.4; 1024 members of 64^2 78 / 107, 100 of 512^2 270 / 580.
+// The 2-D tile serves rotated grids, per-cell fields and planes of 4 GiB.
+int default_tile_config() { return kMarchAutoConfig; }
 
 // the column-marching kernel addresses a plane with 32-bit byte offsets
 bool march_fits(int ny, int pitch, int hi_pitch) {
@@ -371,7 +393,7 @@ bool march_fits(int ny, int pitch, int hi_pitch) {
 int launch_substep(const SubstepArgs& A, int cfg, bool field, hipStream_t s) {
     const bool fits = march_fits(A.ny, A.pitch, A.hi_pitch);
     if (cfg < 0) {
-        cfg = default_tile_config((long long)A.nx * A.ny);
+        cfg = default_tile_config();
         if (cfg >= kFirstMarchConfig && !fits) cfg = kDefaultTileConfig;
     }
     if (cfg >= kNumTileConfigs)
@@ -594,7 +616,7 @@ int gocean_adjoint_set_record_tile_config(int cfg) {
 
 int gocean_adjoint_record_tile_config(void) { return g_record_cfg; }
 
-int gocean_default_tile_config(int nx, int ny) { return default_tile_config((long long)nx * ny); }
+int gocean_default_tile_config(int, int) { return default_tile_config(); }
 
 int gocean_sqrt_newton_check(uint32_t lo_bits, uint32_t hi_bits, unsigned long long* mismatches) {
     clear_error();

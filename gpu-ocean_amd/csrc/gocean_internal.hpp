@@ -22,7 +22,7 @@ extern const int kMarchAutoConfig;
 // configurations kFirstMarchConfig .. kNumTileConfigs-1 are column marching
 constexpr int kFirstMarchConfig = 7;
 // configuration used when the caller passes -1
-int default_tile_config(long long cells);
+int default_tile_config();
 
 int set_error(int code, const char* fmt, ...);
 void clear_error();
@@ -44,7 +44,7 @@ bool march_fits(int ny, int pitch, int hi_pitch);
 // and the rows per strip that fill whole rounds of them
 int resident_waves(const void* kernel);
 int march_stage(int rk_order, int rk_step, float r);
-int march_rows(const int* strips, const int* ny, int n, int resident);
+int march_rows(const int* strips, const int* ny, int n, int resident, int least);
 int launch_substep(const SubstepArgs& A, int cfg, bool field, hipStream_t s);
 // zero-rotation substep that also writes the branch record (A.tape_*)
 int launch_substep_tape(SubstepArgs A, hipStream_t s);

@@ -157,7 +157,7 @@ int gocean_max_dt_static(const gocean_domain_t* d, const float* eta, const float
                          void* stream);
 
 /* Tile configuration (index into gocean_tile_configs; -1, the default: the
- * column-marching kernel from a million cells on, 32x16/512 below) of the
+ * column-marching kernel) of the
  * recording forward substep the adjoint entry points run
  * (gocean_adjoint_record / _segment).  Process-wide; every configuration
  * writes the same record.  An ensemble records with its own configuration
@@ -183,7 +183,8 @@ int gocean_adjoint_reverse_kernel(void);
 int gocean_tile_configs(const char** names, int max);
 /* The configuration a tile_config of -1 selects for an nx x ny domain (or an
  * ensemble whose members average nx*ny cells): the column-marching kernel
- * from a million cells on, the 32x16/512 tile below. */
+ * with balanced rows per strip, whatever the size (planes of 4 GiB or more
+ * take a 2-D tile instead). */
 int gocean_default_tile_config(int nx, int ny);
 
 /* Device self-check of the square root the substep kernels take for wave

@@ -1,0 +1,49 @@
+"""The default configuration (-1) over the sizes its rows-per-strip rule spans:
+a strip of one row on the smallest domains, ragged last strips and rows, and
+more strips than one round of resident waves.  Every configuration gives the
+same bits, so the 2-D tile kernel is the reference."""
+
+import numpy as np
+import pytest
+
+import helpers as H
+from test_gpu_march_paths import _case
+
+pytestmark = pytest.mark.gpu
+
+TILE = 1
+
+
+@pytest.mark.parametrize("nx,ny", [(2, 3), (61, 5), (96, 80), (503, 301), (1030, 517)])
+@pytest.mark.parametrize("bc", [(1, 1, 1, 1), (2, 2, 2, 2), (1, 2, 1, 2)])
+def test_default_equals_tile(nx, ny, bc):
+    print("default config", nx, ny, bc, flush=True)
+    inp, p, Hif, Hm = _case(nx, ny, bc, nx + ny, "land")
+    D = H.DeviceDomain(inp)
+    D.bathymetry_init()
+    out = []
+    for tile in (TILE, -1):
+        h0, h1 = D.state(inp.eta, inp.hu, inp.hv), D.state(inp.eta, inp.hu, inp.hv)
+        D.rk_steps(2, np.float32(0.3), h0, h1, tile=tile)
+        out.append(D.host(h0))
+    for a, b, name in zip(out[0], out[1], ("eta", "hu", "hv")):
+        assert H.normal_equal(a, b), (name, H.diff_report(a, b))
+
+
+def test_default_ensemble_equals_tile():
+    print("default ensemble", flush=True)
+    from SWESimulators import CDKLM16Ensemble, Common
+    ctx = Common.HIPContext()
+    members = []
+    for k, (nx, ny, bc) in enumerate([(2, 2, (1, 1, 1, 1)), (64, 64, (1, 2, 1, 2)), (121, 33, (2, 2, 2, 2)), (59, 260, (2, 1, 2, 1))]):
+        inp, _, _, _ = _case(nx, ny, bc, 40 + k, "deep")
+        members.append(dict(nx=nx, ny=ny, dx=inp.dx, dy=inp.dy, f=inp.f, bc=bc, Hi=inp.Hi, eta=inp.eta, hu=inp.hu,
+                            hv=inp.hv, wind_x=1e-4))
+    states = []
+    for cfg in (TILE, None):
+        ens = CDKLM16Ensemble.CDKLM16Ensemble(ctx, members, dt=0.3, tile_config=cfg)
+        ens.step_n(3)
+        ens.gpu_stream.synchronize()
+        states.append(ens.state[0].cpu().numpy())
+        ens.cleanUp()
+    assert H.normal_equal(*states)
