@@ -198,6 +198,9 @@ class CDKLM16(Simulator.Simulator):
             # dt reduction scratch: [min, courant*min, partial minima...]
             self.dt_scratch = torch.zeros(2 + 1024, dtype=torch.float32, device=dev)
             self.h2 = None
+        # the two results again in pinned host memory, written by the kernel
+        self.dt_pinned = torch.zeros(2, dtype=torch.float32, pin_memory=True)
+        self.dt_result = self.dt_pinned.numpy()
         # texture handles of the reference; the fields above replace them
         self.angle_texref = self.field_tensors[1:] if self.field_tensors else None
         self.coriolis_texref = self.field_tensors[0] if self.field_tensors else None
@@ -215,10 +218,11 @@ class CDKLM16(Simulator.Simulator):
         w.t = float(np.float32(wt))
         ws = self.wind_stress
         if ws.is_uniform():
-            w.x0 = float(np.asarray(ws.X[t0], np.float32).flat[0])
-            w.x1 = float(np.asarray(ws.X[t1], np.float32).flat[0])
-            w.y0 = float(np.asarray(ws.Y[t0], np.float32).flat[0])
-            w.y1 = float(np.asarray(ws.Y[t1], np.float32).flat[0])
+            w.x0 = w.x1 = np.asarray(ws.X[t0], np.float32).item(0)
+            w.y0 = w.y1 = np.asarray(ws.Y[t0], np.float32).item(0)
+            if t1 != t0:
+                w.x1 = np.asarray(ws.X[t1], np.float32).item(0)
+                w.y1 = np.asarray(ws.Y[t1], np.float32).item(0)
             return w
         torch = Common._torch()
         shape = np.asarray(ws.X[0]).shape
@@ -279,6 +283,7 @@ class CDKLM16(Simulator.Simulator):
             self.bathymetry.release()
         self.field_tensors = None
         self.dt_scratch = None
+        self.dt_pinned = self.dt_result = None
         self.h2 = None
         self.gpu_ctx = None
         gc.collect()
@@ -467,10 +472,13 @@ class CDKLM16(Simulator.Simulator):
         taken in double, as NumPy 1.x evaluated ``float * float32``."""
         if courant_number is None:
             courant_number = self.courant_number
-        s = self.max_dt_device(courant_number)
+        gd = self.gpu_data
+        G.check(self.lib.gocean_max_dt_host(self.domain, gd.h0.data.gpudata, gd.hu0.data.gpudata,
+                                            gd.hv0.data.gpudata, self.bathymetry.Bm.data.gpudata,
+                                            float(courant_number), G.ptr(self.dt_scratch),
+                                            self.dt_pinned.data_ptr(), self._stream()), "gocean_max_dt_host")
         self.gpu_stream.synchronize()
-        dt_host = np.float32(s[0].item())
-        self.dt = float(courant_number) * float(dt_host)
+        self.dt = float(courant_number) * float(self.dt_result[0])
 
     def _getMaxTimestepHost(self, courant_number=0.8):
         """Host closed form of the CFL step (CDKLM16.py:741-759)."""

@@ -3,6 +3,7 @@ parameters, stream, wind-stress time interpolation, download/upload/copy."""
 
 from __future__ import annotations
 
+import bisect
 import logging
 from abc import ABCMeta, abstractmethod
 
@@ -56,8 +57,9 @@ class Simulator(object):
         (Simulator.update_wind_stress, Simulator.py:145-223)."""
         ws = self.wind_stress
         t_max_index = len(ws.t) - 1
-        t0_index = max(0, int(np.searchsorted(ws.t, self.t)) - 1)
-        t1_index = min(t_max_index, int(np.searchsorted(ws.t, self.t)))
+        at = bisect.bisect_left(ws.t, self.t)
+        t0_index = max(0, at - 1)
+        t1_index = min(t_max_index, at)
         new_t0 = ws.t[t0_index]
         new_t1 = ws.t[t1_index]
         elapsed_since_t0 = (self.t - new_t0)

@@ -67,6 +67,8 @@ PROTOTYPES = [
     ("gocean_periodic_bc", c_int, [ctypes.POINTER(Domain), c_void_p, c_void_p, c_void_p, c_void_p]),
     ("gocean_max_dt", c_int,
      [ctypes.POINTER(Domain), c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p]),
+    ("gocean_max_dt_host", c_int,
+     [ctypes.POINTER(Domain), c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p]),
     ("gocean_max_dt_static", c_int,
      [ctypes.POINTER(Domain), c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p]),
     ("gocean_default_tile_config", c_int, [c_int, c_int]),

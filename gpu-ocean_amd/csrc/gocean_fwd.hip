@@ -555,8 +555,10 @@ __global__ __launch_bounds__(kDtThreads) void k_dt_partial(const float* eta, con
     if (threadIdx.x == 0) partial[blockIdx.x] = m;
 }
 
+// host: the same two values in host memory the device can write (pinned), or
+// NULL; visible there once the stream has been synchronised
 __global__ __launch_bounds__(kDtThreads) void k_dt_final(const float* partial, int n, float courant,
-                                                         float* out) {
+                                                         float* out, float* host) {
     __shared__ float red[kDtThreads / 64];
     float m = 1.0e5f;
     for (int k = threadIdx.x; k < n; k += blockDim.x) m = fminf(m, partial[k]);
@@ -564,17 +566,18 @@ __global__ __launch_bounds__(kDtThreads) void k_dt_final(const float* partial, i
     if (threadIdx.x == 0) {
         out[0] = m;
         out[1] = courant > 0.0f ? courant * m : m;
+        if (host) { host[0] = m; host[1] = out[1]; }
     }
 }
 
 int max_dt_partials(const gocean_domain_t* d) { return d->ny < kDtBlocks ? d->ny : kDtBlocks; }
 
 int max_dt_into(const gocean_domain_t* d, const float* eta, const float* hu, const float* hv,
-                const float* Hm, float courant, float* partial, float* out, hipStream_t s) {
+                const float* Hm, float courant, float* partial, float* out, hipStream_t s, float* host) {
     const int nb = max_dt_partials(d);
     hipLaunchKernelGGL(k_dt_partial, dim3(nb), dim3(kDtThreads), 0, s, eta, hu, hv, Hm, d->nx,
                        d->ny, d->pitch, d->dx, d->dy, d->g, d->land_value, partial);
-    hipLaunchKernelGGL(k_dt_final, dim3(1), dim3(kDtThreads), 0, s, partial, nb, courant, out);
+    hipLaunchKernelGGL(k_dt_final, dim3(1), dim3(kDtThreads), 0, s, partial, nb, courant, out, host);
     return check_launch("max dt launch");
 }
 
@@ -582,6 +585,67 @@ int max_dt(const gocean_domain_t* d, const float* eta, const float* hu, const fl
            const float* Hm, float courant, float* out, hipStream_t s) {
     return max_dt_into(d, eta, hu, hv, Hm, courant, out + 2, out, s);
 }
+
+namespace {
+
+// eta, hu, hv of one state buffer
+struct State {
+    const float *eta, *hu, *hv;
+    bool complete() const { return eta && hu && hv; }
+};
+
+// the arguments every stage of a call shares
+int common_args(const gocean_domain_t* d, float dt, const float* dt_dev, const float* Hi,
+                const gocean_fields_t* fields, const gocean_wind_t* wind, SubstepArgs& A, bool& field) {
+    if (!Hi) return set_error(GOCEAN_EINVAL, "state/bathymetry pointer is NULL");
+    fill_args(d, A);
+    A.Hi = Hi;
+    A.dt = dt;
+    A.dt_dev = dt_dev;
+    field = false;
+    if (fields && (fields->f || fields->north_x || fields->north_y)) {
+        if (!fields->f || !fields->north_x || !fields->north_y)
+            return set_error(GOCEAN_EINVAL, "per-cell fields must give f, north_x and north_y together");
+        A.f_field = fields->f; A.nx_field = fields->north_x; A.ny_field = fields->north_y;
+        field = true;
+    }
+    if (wind) {
+        A.wind_x = wind_lerp(wind->t, wind->x0, wind->x1);
+        A.wind_y = wind_lerp(wind->t, wind->y0, wind->y1);
+        if (wind->grid) {
+            if (wind->grid_nx < 1 || wind->grid_ny < 1)
+                return set_error(GOCEAN_EINVAL, "wind grid %d x %d: both sides must be >= 1",
+                                 wind->grid_nx, wind->grid_ny);
+            A.wind_grid = wind->grid;
+            A.wind_wx = wind->grid_nx;
+            A.wind_wy = wind->grid_ny;
+            A.wind_t = wind->t;
+        }
+    }
+    return 0;
+}
+
+// the stage's own: buffers (Q^n is read from the outputs where not given)
+int stage_args(const gocean_domain_t* d, int rk_step, const State& in, const State& qn, const State& out,
+               SubstepArgs& A) {
+    if (!in.complete() || !out.complete())
+        return set_error(GOCEAN_EINVAL, "state/bathymetry pointer is NULL");
+    if (rk_step < 0 || rk_step >= d->rk_order)
+        return set_error(GOCEAN_EINVAL, "rk_step %d invalid for rk_order %d", rk_step, d->rk_order);
+    if (in.eta == out.eta || in.hu == out.hu || in.hv == out.hv)
+        return set_error(GOCEAN_EINVAL, "input and output state must not alias");
+    A.eta_in = in.eta; A.hu_in = in.hu; A.hv_in = in.hv;
+    A.eta_out = const_cast<float*>(out.eta);
+    A.hu_out = const_cast<float*>(out.hu);
+    A.hv_out = const_cast<float*>(out.hv);
+    A.eta_qn = qn.eta ? qn.eta : out.eta;
+    A.hu_qn = qn.hu ? qn.hu : out.hu;
+    A.hv_qn = qn.hv ? qn.hv : out.hv;
+    A.set_rk_step(rk_step);
+    return 0;
+}
+
+}  // namespace
 
 }  // namespace gocean
 
@@ -679,6 +743,14 @@ int gocean_max_dt(const gocean_domain_t* d, const float* eta, const float* hu, c
     return max_dt(d, eta, hu, hv, Hm, courant, out_dev, (hipStream_t)stream);
 }
 
+int gocean_max_dt_host(const gocean_domain_t* d, const float* eta, const float* hu, const float* hv, const float* Hm,
+                       float courant, float* out_dev, float* out_host, void* stream) {
+    clear_error();
+    if (int e = validate_domain(d)) return e;
+    if (!eta || !hu || !hv || !Hm || !out_dev || !out_host) return set_error(GOCEAN_EINVAL, "NULL pointer");
+    return max_dt_into(d, eta, hu, hv, Hm, courant, out_dev + 2, out_dev, (hipStream_t)stream, out_host);
+}
+
 int gocean_cdklm_substep(const gocean_domain_t* d, float dt, const float* dt_dev, int rk_step,
                          const float* eta_in, const float* hu_in, const float* hv_in,
                          const float* eta_qn, const float* hu_qn, const float* hv_qn,
@@ -687,46 +759,16 @@ int gocean_cdklm_substep(const gocean_domain_t* d, float dt, const float* dt_dev
                          int tile_config, void* stream) {
     clear_error();
     if (int e = validate_domain(d)) return e;
-    if (!eta_in || !hu_in || !hv_in || !eta_out || !hu_out || !hv_out || !Hi)
-        return set_error(GOCEAN_EINVAL, "state/bathymetry pointer is NULL");
-    if (rk_step < 0 || rk_step >= d->rk_order)
-        return set_error(GOCEAN_EINVAL, "rk_step %d invalid for rk_order %d", rk_step, d->rk_order);
-    if (eta_in == eta_out || hu_in == hu_out || hv_in == hv_out)
-        return set_error(GOCEAN_EINVAL, "input and output state must not alias");
+    const State in{eta_in, hu_in, hv_in}, qn{eta_qn, hu_qn, hv_qn}, out{eta_out, hu_out, hv_out};
     SubstepArgs A;
-    fill_args(d, A);
-    A.eta_in = eta_in; A.hu_in = hu_in; A.hv_in = hv_in;
-    A.eta_out = eta_out; A.hu_out = hu_out; A.hv_out = hv_out;
-    A.eta_qn = eta_qn ? eta_qn : eta_out;
-    A.hu_qn = hu_qn ? hu_qn : hu_out;
-    A.hv_qn = hv_qn ? hv_qn : hv_out;
-    A.Hi = Hi;
-    A.dt = dt;
-    A.dt_dev = dt_dev;
-    A.set_rk_step(rk_step);
     bool field = false;
-    if (fields && (fields->f || fields->north_x || fields->north_y)) {
-        if (!fields->f || !fields->north_x || !fields->north_y)
-            return set_error(GOCEAN_EINVAL, "per-cell fields must give f, north_x and north_y together");
-        A.f_field = fields->f; A.nx_field = fields->north_x; A.ny_field = fields->north_y;
-        field = true;
-    }
-    if (wind) {
-        A.wind_x = wind_lerp(wind->t, wind->x0, wind->x1);
-        A.wind_y = wind_lerp(wind->t, wind->y0, wind->y1);
-        if (wind->grid) {
-            if (wind->grid_nx < 1 || wind->grid_ny < 1)
-                return set_error(GOCEAN_EINVAL, "wind grid %d x %d: both sides must be >= 1",
-                                 wind->grid_nx, wind->grid_ny);
-            A.wind_grid = wind->grid;
-            A.wind_wx = wind->grid_nx;
-            A.wind_wy = wind->grid_ny;
-            A.wind_t = wind->t;
-        }
-    }
+    if (int e = common_args(d, dt, dt_dev, Hi, fields, wind, A, field)) return e;
+    if (int e = stage_args(d, rk_step, in, qn, out, A)) return e;
     return launch_substep(A, tile_config, field, (hipStream_t)stream);
 }
 
+// The arguments of the stages are formed once for all n_steps: only launches
+// are left in the loop.
 int gocean_rk_steps(const gocean_domain_t* d, int n_steps, float dt, const float* dt_dev,
                     float* eta0, float* hu0, float* hv0, float* eta1, float* hu1, float* hv1,
                     float* eta2, float* hu2, float* hv2, const float* Hi,
@@ -740,37 +782,29 @@ int gocean_rk_steps(const gocean_domain_t* d, int n_steps, float dt, const float
     if (d->rk_order == 1 && n_steps % 2 != 0)
         return set_error(GOCEAN_EINVAL,
                          "rk_order 1 swaps buffers every step; call with an even n_steps");
-    for (int n = 0; n < n_steps; ++n) {
-        int e = 0;
-        if (d->rk_order == 2) {
-            e = gocean_cdklm_substep(d, dt, dt_dev, 0, eta0, hu0, hv0, nullptr, nullptr, nullptr,
-                                     eta1, hu1, hv1, Hi, fields, wind, tile_config, stream);
-            if (!e)
-                e = gocean_cdklm_substep(d, dt, dt_dev, 1, eta1, hu1, hv1, nullptr, nullptr, nullptr,
-                                         eta0, hu0, hv0, Hi, fields, wind, tile_config, stream);
-        } else if (d->rk_order == 1) {
-            // Euler: h0 -> h1, then the caller's buffers swap; two steps
-            // bring the state back into h0.
-            if (n % 2 == 0)
-                e = gocean_cdklm_substep(d, dt, dt_dev, 0, eta0, hu0, hv0, nullptr, nullptr, nullptr,
-                                         eta1, hu1, hv1, Hi, fields, wind, tile_config, stream);
-            else
-                e = gocean_cdklm_substep(d, dt, dt_dev, 0, eta1, hu1, hv1, nullptr, nullptr, nullptr,
-                                         eta0, hu0, hv0, Hi, fields, wind, tile_config, stream);
-        } else {
-            // SSP-RK3; the middle stage goes to the third buffer instead of
-            // overwriting its own input as the reference does
-            e = gocean_cdklm_substep(d, dt, dt_dev, 0, eta0, hu0, hv0, nullptr, nullptr, nullptr,
-                                     eta1, hu1, hv1, Hi, fields, wind, tile_config, stream);
-            if (!e)
-                e = gocean_cdklm_substep(d, dt, dt_dev, 1, eta1, hu1, hv1, eta0, hu0, hv0, eta2, hu2,
-                                         hv2, Hi, fields, wind, tile_config, stream);
-            if (!e)
-                e = gocean_cdklm_substep(d, dt, dt_dev, 2, eta2, hu2, hv2, nullptr, nullptr, nullptr,
-                                         eta0, hu0, hv0, Hi, fields, wind, tile_config, stream);
-        }
-        if (e) return e;
+    if (n_steps == 0) return 0;
+    const State h0{eta0, hu0, hv0}, h1{eta1, hu1, hv1}, h2{eta2, hu2, hv2}, none{nullptr, nullptr, nullptr};
+    // stage k of a step; Euler (order 1): h0 -> h1, then the caller's buffers
+    // swap, and two steps bring the state back into h0; SSP-RK3: the middle
+    // stage goes to the third buffer instead of overwriting its own input as
+    // the reference does
+    struct Stage { int rk_step; State in, qn, out; };
+    const Stage euler[2] = {{0, h0, none, h1}, {0, h1, none, h0}};
+    const Stage rk2[2] = {{0, h0, none, h1}, {1, h1, none, h0}};
+    const Stage rk3[3] = {{0, h0, none, h1}, {1, h1, h0, h2}, {2, h2, none, h0}};
+    const Stage* stages = d->rk_order == 1 ? euler : d->rk_order == 2 ? rk2 : rk3;
+    const int n_stages = d->rk_order == 3 ? 3 : 2;
+    const int rounds = d->rk_order == 1 ? n_steps / 2 : n_steps;
+    SubstepArgs A[3];
+    bool field = false;
+    if (int e = common_args(d, dt, dt_dev, Hi, fields, wind, A[0], field)) return e;
+    for (int k = n_stages - 1; k >= 0; --k) {
+        A[k] = A[0];
+        if (int e = stage_args(d, stages[k].rk_step, stages[k].in, stages[k].qn, stages[k].out, A[k])) return e;
     }
+    for (int n = 0; n < rounds; ++n)
+        for (int k = 0; k < n_stages; ++k)
+            if (int e = launch_substep(A[k], tile_config, field, (hipStream_t)stream)) return e;
     return 0;
 }
 

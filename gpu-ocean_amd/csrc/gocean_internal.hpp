@@ -55,7 +55,7 @@ int periodic_bc(const gocean_domain_t* d, float* e, float* u, float* v, hipStrea
 constexpr int kMaxDtPartials = 1024;
 int max_dt_partials(const gocean_domain_t* d);
 int max_dt_into(const gocean_domain_t* d, const float* eta, const float* hu, const float* hv,
-                const float* Hm, float courant, float* partial, float* out, hipStream_t s);
+                const float* Hm, float courant, float* partial, float* out, hipStream_t s, float* host = nullptr);
 int max_dt(const gocean_domain_t* d, const float* eta, const float* hu, const float* hv,
            const float* Hm, float courant, float* out, hipStream_t s);
 // substep-adjoint kernel of the reverse entry points (0 tile, 1 marching)

@@ -144,6 +144,13 @@ int gocean_max_dt(const gocean_domain_t* d, const float* eta, const float* hu,
                   const float* hv, const float* Hm, float courant, float* out_dev,
                   void* stream);
 
+/* gocean_max_dt that also writes its two results to out_host, pinned host
+ * memory the device can write; valid there once the stream has been
+ * synchronised, without a copy.  Same results, bit for bit. */
+int gocean_max_dt_host(const gocean_domain_t* d, const float* eta, const float* hu,
+                       const float* hv, const float* Hm, float courant, float* out_dev,
+                       float* out_host, void* stream);
+
 /* gocean_max_dt without the caller's partial-minima buffer: out_dev holds
  * just the two results, and the partial minima go to a static device array of
  * the library (1024 floats, one copy per GPU, kept until the process ends).

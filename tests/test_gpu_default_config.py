@@ -47,3 +47,21 @@ def test_default_ensemble_equals_tile():
         states.append(ens.state[0].cpu().numpy())
         ens.cleanUp()
     assert H.normal_equal(*states)
+
+
+@pytest.mark.parametrize("nx,ny", [(2, 2), (61, 5), (300, 1030)])
+def test_max_dt_in_host_memory(nx, ny):
+    """The minima the kernel writes to pinned host memory are the device's."""
+    print("max dt host", nx, ny, flush=True)
+    import torch
+    inp, p, Hif, Hm = _case(nx, ny, (1, 2, 1, 2), nx, "film")
+    D = H.DeviceDomain(inp)
+    D.bathymetry_init()
+    h = D.state(inp.eta, inp.hu, inp.hv)
+    pinned = torch.zeros(2, pin_memory=True)
+    D.G.check(D.lib.gocean_max_dt_host(D.dom, h[0].data_ptr(), h[1].data_ptr(), h[2].data_ptr(), D.Hm.data_ptr(), 0.7,
+                                       D.scratch.data_ptr(), pinned.data_ptr(), None), "max_dt_host")
+    torch.cuda.synchronize()
+    got = pinned.numpy().copy()
+    assert np.array_equal(got, D.scratch[:2].cpu().numpy())
+    assert np.array_equal(got, D.max_dt(h, courant=0.7))
