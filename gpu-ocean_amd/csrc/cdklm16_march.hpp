@@ -569,6 +569,11 @@ __device__ __forceinline__ void march_strip(const SubstepArgs& A, int sx, int sy
         float ea = 0.0f, ha = 0.0f, va = 0.0f;
         if (later) { ea = ld(r_eqn, ocl, rj); ha = ld(r_uqn, ocl, rj); va = ld(r_vqn, ocl, rj); }
 
+        // the gridded wind's 16 texels of the lane's cell: in flight until
+        // the sources at the end of the row
+        WindCell wcell;
+        if (wgrid) wcell = wind_grid_load(A.wind_grid, A.wind_wx, A.wind_wy, wax, wind_axis(j, ny, A.wind_wy));
+
         // ---- x slope centre of row j (neighbours by lane exchange) ----
         const float el = from_left(cj.E), er = from_right(cj.E);
         const float ul = from_left(cj.U), ur = from_right(cj.U);
@@ -662,9 +667,7 @@ __device__ __forceinline__ void march_strip(const SubstepArgs& A, int sx, int sy
             // one fma, and (g m) (0.5 D) = (0.5 g m) D
             auto sources = [&](float hu, float hv, float& st1, float& st2) {
                 float X = A.wind_x, Y = A.wind_y;
-                if (wgrid)
-                    wind_grid_at(A.wind_grid, A.wind_wx, A.wind_wy, A.wind_t, wax, wind_axis(j, ny, A.wind_wy),
-                                 X, Y);
+                if (wgrid) wind_grid_value(wcell, A.wind_t, X, Y);
                 const float eta_we = (ec - T) + (ec + T);
                 const float eta_sn = (ec + Sj) + (ec - Sj);
                 const float b1 = (K.half_g * fmaf(0.5f, eta_we, Hm)) * (He2 - Hw2);

@@ -124,23 +124,40 @@ __device__ __forceinline__ WindAxis wind_axis(int ti, int n, int w) {
     return o;
 }
 
-// bilinear value of one wind plane (row length w) at (ax, ay)
-__device__ __forceinline__ float wind_bilinear(const float* F, int w, const WindAxis& ax, const WindAxis& ay) {
-    const float a = ax.a, b = ay.a;
+// the four texels of one wind plane (row length w) around (ax, ay)
+struct WindTexels {
+    float c00, c01, c10, c11;      // [y][x]
+};
+
+__device__ __forceinline__ WindTexels wind_texels(const float* F, int w, const WindAxis& ax, const WindAxis& ay) {
     const float* r0 = F + (size_t)ay.i0 * w;
     const float* r1 = F + (size_t)ay.i1 * w;
-    return ((((1.0f - a) * (1.0f - b)) * r0[ax.i0] + (a * (1.0f - b)) * r0[ax.i1])
-            + ((1.0f - a) * b) * r1[ax.i0]) + (a * b) * r1[ax.i1];
+    return WindTexels{r0[ax.i0], r0[ax.i1], r1[ax.i0], r1[ax.i1]};
 }
 
-// gridded wind stress (X, Y) of one cell, interpolated in time
-__device__ __forceinline__ void wind_grid_at(const float* grid, int wx, int wy, float wt,
-                                             const WindAxis& ax, const WindAxis& ay, float& X, float& Y) {
+__device__ __forceinline__ float wind_bilinear(const WindTexels& t, float a, float b) {
+    return ((((1.0f - a) * (1.0f - b)) * t.c00 + (a * (1.0f - b)) * t.c01)
+            + ((1.0f - a) * b) * t.c10) + (a * b) * t.c11;
+}
+
+// gridded wind stress of one cell: the texels of the X0, X1, Y0, Y1 planes,
+// and from them (X, Y), interpolated in time.  Apart, so that a caller can
+// have the loads in flight while it computes.
+struct WindCell {
+    WindTexels x0, x1, y0, y1;
+    float a, b;
+};
+
+__device__ __forceinline__ WindCell wind_grid_load(const float* grid, int wx, int wy, const WindAxis& ax,
+                                                   const WindAxis& ay) {
     const size_t pl = (size_t)wx * wy;
-    const float x0 = wind_bilinear(grid, wx, ax, ay), x1 = wind_bilinear(grid + pl, wx, ax, ay);
-    const float y0 = wind_bilinear(grid + 2 * pl, wx, ax, ay), y1 = wind_bilinear(grid + 3 * pl, wx, ax, ay);
-    X = wind_lerp(wt, x0, x1);
-    Y = wind_lerp(wt, y0, y1);
+    return WindCell{wind_texels(grid, wx, ax, ay), wind_texels(grid + pl, wx, ax, ay),
+                    wind_texels(grid + 2 * pl, wx, ax, ay), wind_texels(grid + 3 * pl, wx, ax, ay), ax.a, ay.a};
+}
+
+__device__ __forceinline__ void wind_grid_value(const WindCell& w, float wt, float& X, float& Y) {
+    X = wind_lerp(wt, wind_bilinear(w.x0, w.a, w.b), wind_bilinear(w.x1, w.a, w.b));
+    Y = wind_lerp(wt, wind_bilinear(w.y0, w.a, w.b), wind_bilinear(w.y1, w.a, w.b));
 }
 
 // 1/d - RN(1/d), rounded: the double quotient is off by 2^-53 relative, the
@@ -885,8 +902,8 @@ __device__ __forceinline__ void cdklm_tile(const SubstepArgs& A, int tile_x, int
             float X = A.wind_x, Y = A.wind_y;
             // the recording variant serves the adjoint, which takes uniform wind
             if (!TAPE && A.wind_grid)
-                wind_grid_at(A.wind_grid, A.wind_wx, A.wind_wy, A.wind_t, wind_axis(C, nx, A.wind_wx),
-                             wind_axis(R, ny, A.wind_wy), X, Y);
+                wind_grid_value(wind_grid_load(A.wind_grid, A.wind_wx, A.wind_wy, wind_axis(C, nx, A.wind_wx),
+                                               wind_axis(R, ny, A.wind_wy)), A.wind_t, X, Y);
             const float RHxp = 0.5f * (S.Hi[rr][cc + 1] + S.Hi[rr + 1][cc + 1]);
             const float RHxm = 0.5f * (S.Hi[rr][cc] + S.Hi[rr + 1][cc]);
             const float RHyp = 0.5f * (S.Hi[rr + 1][cc] + S.Hi[rr + 1][cc + 1]);
