@@ -198,9 +198,7 @@ class CDKLM16(Simulator.Simulator):
             # dt reduction scratch: [min, courant*min, partial minima...]
             self.dt_scratch = torch.zeros(2 + 1024, dtype=torch.float32, device=dev)
             self.h2 = None
-        # the two results again in pinned host memory, written by the kernel
-        self.dt_pinned = torch.zeros(2, dtype=torch.float32, pin_memory=True)
-        self.dt_result = self.dt_pinned.numpy()
+        self.dt_pinned = self.dt_result = None
         # texture handles of the reference; the fields above replace them
         self.angle_texref = self.field_tensors[1:] if self.field_tensors else None
         self.coriolis_texref = self.field_tensors[0] if self.field_tensors else None
@@ -472,6 +470,10 @@ class CDKLM16(Simulator.Simulator):
         taken in double, as NumPy 1.x evaluated ``float * float32``."""
         if courant_number is None:
             courant_number = self.courant_number
+        if self.dt_pinned is None:
+            # the two results again in pinned host memory, written by the kernel
+            self.dt_pinned = Common._torch().zeros(2, dtype=Common._torch().float32, pin_memory=True)
+            self.dt_result = self.dt_pinned.numpy()
         gd = self.gpu_data
         G.check(self.lib.gocean_max_dt_host(self.domain, gd.h0.data.gpudata, gd.hu0.data.gpudata,
                                             gd.hv0.data.gpudata, self.bathymetry.Bm.data.gpudata,

@@ -213,6 +213,10 @@ __host__ __device__ __forceinline__ float minmod_slope(float l, float c, float r
     return minmod_raw((c - l) * theta, (r - l) * 0.5f, (r - c) * theta);
 }
 
+__device__ __forceinline__ float minmod3_slope(float l, float c, float r, float theta) {
+    return minmod3((c - l) * theta, (r - l) * 0.5f, (r - c) * theta);
+}
+
 // which candidate minmod_raw(b, c, f) returns: 0, 1, 2, or 3 when the sign
 // bits disagree (result zero).  Ties pick the first; the value is the same.
 __host__ __device__ __forceinline__ uint32_t minmod_sel(float b, float c, float f) {
@@ -281,6 +285,8 @@ __device__ __forceinline__ float div_r(float n, float d, float r) {
 // is correctly rounded for most divisors; the host enables it (SubstepArgs
 // fast_arith()) only for divisors for which it has checked every float
 // significand of n (fast_arith_exact in gocean_fwd.hip); otherwise div_r runs.
+// Quotients below 2^-101, where n l is subnormal, can be one unit in the last
+// place off.
 template <bool FAST>
 __device__ __forceinline__ float div_k(float n, float d, float r, float l) {
     if constexpr (FAST) return fmaf(n, r, n * l);
@@ -413,6 +419,12 @@ struct TileSmem {
     float F2[FIELD ? 3 : 1][FIELD ? BH : 1][FIELD ? BW + 1 : 1];
     float G2[FIELD ? 3 : 1][FIELD ? BH + 1 : 1][FIELD ? BW : 1];
 };
+
+// Waves per SIMD a tile kernel's registers are held to: 512-thread tiles take 8
+// (four workgroups per CU) at the price of a few spills into vector-register
+// lanes, where the LDS allows it; the field mode's 53 KB allow 6.
+template <int NT, int MODE>
+constexpr int tile_waves() { return NT < 512 ? 1 : MODE == kModeField ? 6 : 8; }
 
 // Map a workgroup index to a tile index so that each of the 8 XCDs (which
 // receive workgroups round-robin) works on one contiguous band of tiles and
@@ -584,8 +596,8 @@ __device__ __forceinline__ void cdklm_tile(const SubstepArgs& A, int tile_x, int
             const float el = S.E[rr][cc - 1], ec = S.E[rr][cc], er = S.E[rr][cc + 1];
             const float ul = S.U[rr][cc - 1], uc = S.U[rr][cc], ur = S.U[rr][cc + 1];
             float vl = S.V[rr][cc - 1], vc = S.V[rr][cc], vr = S.V[rr][cc + 1];
-            S.Ux[j][i] = minmod_slope(ul, uc, ur, K.theta);
-            S.Vx[j][i] = minmod_slope(vl, vc, vr, K.theta);
+            S.Ux[j][i] = minmod3_slope(ul, uc, ur, K.theta);
+            S.Vx[j][i] = minmod3_slope(vl, vc, vr, K.theta);
             const float vc_raw = vc;
             const bool flip_c = ghost_col_flip(C);
             if (ghost_col_flip(C - 1)) vl = -vl;
@@ -605,7 +617,7 @@ __device__ __forceinline__ void cdklm_tile(const SubstepArgs& A, int tile_x, int
             const float bw_ = K.theta_g * ((ec - el) - K.vdx * (fv_c + fv_l));
             const float ce_ = K.half_g * ((er - el) - K.vdx * ((fv_r + 2.0f * fv_c) + fv_l));
             const float fw_ = K.theta_g * ((er - ec) - K.vdx * (fv_c + fv_r));
-            float Kx = minmod_raw(bw_, ce_, fw_);
+            float Kx = minmod3(bw_, ce_, fw_);
             // positivity adjustment; the reference flips v only in west ghost
             // column 1 here (its east test, bx+k > NX+2, never hits a column
             // an interior cell reads)
@@ -646,8 +658,8 @@ __device__ __forceinline__ void cdklm_tile(const SubstepArgs& A, int tile_x, int
             const float el = S.E[rr - 1][cc], ec = S.E[rr][cc], eu = S.E[rr + 1][cc];
             float ul = S.U[rr - 1][cc], uc = S.U[rr][cc], uu = S.U[rr + 1][cc];
             const float vl = S.V[rr - 1][cc], vc = S.V[rr][cc], vu = S.V[rr + 1][cc];
-            S.Uy[j][i] = minmod_slope(ul, uc, uu, K.theta);
-            S.Vy[j][i] = minmod_slope(vl, vc, vu, K.theta);
+            S.Uy[j][i] = minmod3_slope(ul, uc, uu, K.theta);
+            S.Vy[j][i] = minmod3_slope(vl, vc, vu, K.theta);
             const float uc_raw = uc;
             const bool flip_c = ghost_row_flip(R);
             if (ghost_row_flip(R - 1)) ul = -ul;
@@ -668,7 +680,7 @@ __device__ __forceinline__ void cdklm_tile(const SubstepArgs& A, int tile_x, int
             const float bw_ = K.theta_g * ((ec - el) + K.udy * (fu_c + fu_l));
             const float ce_ = K.half_g * ((eu - el) + K.udy * ((fu_u + 2.0f * fu_c) + fu_l));
             const float fw_ = K.theta_g * ((eu - ec) + K.udy * (fu_c + fu_u));
-            float Ly = minmod_raw(bw_, ce_, fw_);
+            float Ly = minmod3(bw_, ce_, fw_);
             const bool flip_a = wS && R < 2;
             const float dfc = K.dy * fc;
             const float dyfu = dfc * (flip_a ? -uc_raw : uc_raw);
@@ -736,13 +748,19 @@ __device__ __forceinline__ void cdklm_tile(const SubstepArgs& A, int tile_x, int
                         const float hm = fmaxf(0.0f, (eta_m + H_face) + div_r(Km + dfm * vmn, K.two_g, K.r_two_g));
                         cu_flux(hm, Rmx, Rmy, hp, Rpx, Rpy, K, Fx, Fy, Fz);
                     }
+                    // the other cell's north vector: the same face where the
+                    // two are equal (a varying f alone, a grid rotated as a
+                    // whole)
                     if constexpr (FIELD) {
                         const float n_x = nxcell(rr, cp), n_y = nycell(rr, cp);
-                        const float vpn = up * n_x + vp * n_y;
-                        const float vmn = um * n_x + vm * n_y;
-                        const float hp = fmaxf(0.0f, (eta_p + H_face) - div_r(Kp + dfp * vpn, K.two_g, K.r_two_g));
-                        const float hm = fmaxf(0.0f, (eta_m + H_face) + div_r(Km + dfm * vmn, K.two_g, K.r_two_g));
-                        cu_flux(hm, Rmx, Rmy, hp, Rpx, Rpy, K, Fx2, Fy2, Fz2);
+                        Fx2 = Fx; Fy2 = Fy; Fz2 = Fz;
+                        if (n_x != nxcell(rr, cm) || n_y != nycell(rr, cm)) {
+                            const float vpn = up * n_x + vp * n_y;
+                            const float vmn = um * n_x + vm * n_y;
+                            const float hp = fmaxf(0.0f, (eta_p + H_face) - div_r(Kp + dfp * vpn, K.two_g, K.r_two_g));
+                            const float hm = fmaxf(0.0f, (eta_m + H_face) + div_r(Km + dfm * vmn, K.two_g, K.r_two_g));
+                            cu_flux(hm, Rmx, Rmy, hp, Rpx, Rpy, K, Fx2, Fy2, Fz2);
+                        }
                     }
                 }
             }
@@ -788,13 +806,16 @@ __device__ __forceinline__ void cdklm_tile(const SubstepArgs& A, int tile_x, int
                     }
                     if constexpr (FIELD) {
                         const float e_x = nycell(rp, cc), e_y = -nxcell(rp, cc);
-                        const float upe = up * e_x + vp * e_y;
-                        const float ume = um * e_x + vm * e_y;
-                        const float hp = fmaxf(0.0f, (eta_p + H_face) - div_r(Lp - dfp * upe, K.two_g, K.r_two_g));
-                        const float hm = fmaxf(0.0f, (eta_m + H_face) + div_r(Lm - dfm * ume, K.two_g, K.r_two_g));
-                        float a, b, c;
-                        cu_flux(hm, Rmy, Rmx, hp, Rpy, Rpx, K, a, b, c);
-                        Gx2 = a; Gy2 = c; Gz2 = b;
+                        Gx2 = Gx; Gy2 = Gy; Gz2 = Gz;
+                        if (e_x != nycell(rm, cc) || e_y != -nxcell(rm, cc)) {
+                            const float upe = up * e_x + vp * e_y;
+                            const float ume = um * e_x + vm * e_y;
+                            const float hp = fmaxf(0.0f, (eta_p + H_face) - div_r(Lp - dfp * upe, K.two_g, K.r_two_g));
+                            const float hm = fmaxf(0.0f, (eta_m + H_face) + div_r(Lm - dfm * ume, K.two_g, K.r_two_g));
+                            float a, b, c;
+                            cu_flux(hm, Rmy, Rmx, hp, Rpy, Rpx, K, a, b, c);
+                            Gx2 = a; Gy2 = c; Gz2 = b;
+                        }
                     }
                 }
             }

@@ -100,7 +100,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
 }
 
 template <int BW, int BH, int NT, int MODE>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 512 ? 8 : 1))) void k_ens_substep(EnsLaunch L) {
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(tile_waves<NT, MODE>()))) void k_ens_substep(EnsLaunch L) {
     __shared__ TileSmem<BW, BH, MODE> S;
     const int t = xcd_band(blockIdx.x, gridDim.x);
     const int m = L.tile_member[t];
@@ -521,9 +521,9 @@ static int ens_launch(const gocean_ensemble* E, EnsLaunch L, hipStream_t s) {
     L.tile_member = E->d_tile_member;
     L.n_tiles = E->n_tiles;
     if (E->mode == kModeField) {
-        ens_launch_t<32, 8, 256, kModeField>(L, s);
+        ens_launch_t<kGeneralBW, kGeneralBH, kGeneralNT, kModeField>(L, s);
     } else if (E->mode == kModeConst) {
-        ens_launch_t<32, 8, 256, kModeConst>(L, s);
+        ens_launch_t<kGeneralBW, kGeneralBH, kGeneralNT, kModeConst>(L, s);
     } else {
         switch (E->cfg) {
             case 0: ens_launch_t<32, 8, 256, kModeZero>(L, s); break;
@@ -625,7 +625,7 @@ int gocean_ensemble_create(const gocean_member_t* members, int n, int tile_confi
         E->fast_arith = E->fast_arith && fast_arith_exact(d.g, d.dx, d.dy, d.depth_cutoff);
         E->friction = std::max(E->friction, d.r);
     }
-    const TileConfig& tc = (E->mode == kModeZero) ? kTileConfigs[E->cfg] : kTileConfigs[0];
+    const TileConfig& tc = (E->mode == kModeZero) ? kTileConfigs[E->cfg] : kGeneralTile;
     E->bw = tc.bw; E->bh = tc.bh; E->nt = tc.nt;
     if (E->bh == 0) {
         std::vector<EnsMember> shape(n);
@@ -697,7 +697,7 @@ int gocean_ensemble_set_tile_config(gocean_ensemble_t* E, int tile_config) {
     // work already queued may still read the old tables
     if (hipDeviceSynchronize() != hipSuccess) return check_launch("ensemble tile configuration");
     E->cfg = tile_config;
-    const TileConfig& tc = (E->mode == kModeZero) ? kTileConfigs[E->cfg] : kTileConfigs[0];
+    const TileConfig& tc = (E->mode == kModeZero) ? kTileConfigs[E->cfg] : kGeneralTile;
     E->bw = tc.bw; E->bh = tc.bh; E->nt = tc.nt;
     if (E->bh == 0) E->bh = ens_march_rows(E->members, E->fast_arith);
     std::vector<int> tile_member;

@@ -173,7 +173,7 @@ const int kMarchAutoConfig = 9;
 // price of a few scalar-register spills into vector-register lanes; measured
 // faster than the 7 waves the registers otherwise allow
 template <int BW, int BH, int NT, int MODE>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 512 ? 8 : 1))) void k_substep(SubstepArgs A) {
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(tile_waves<NT, MODE>()))) void k_substep(SubstepArgs A) {
     __shared__ TileSmem<BW, BH, MODE> S;
     const int t = xcd_band(blockIdx.x, gridDim.x);
     const int ty = t / A.tiles_x, tx = t - ty * A.tiles_x;
@@ -402,10 +402,11 @@ int launch_substep(const SubstepArgs& A, int cfg, bool field, hipStream_t s) {
         return set_error(GOCEAN_EINVAL, "tile configuration %d (column marching) needs planes below 4 GiB", cfg);
     const int mode = substep_mode(A, field);
     if (mode == kModeField) {
-        // per-cell Coriolis / north fields: one general configuration
-        launch_substep_t<32, 8, 256, kModeField>(A, s);
+        // per-cell Coriolis / north fields, and rotated grids below: one
+        // general configuration (kGeneralBW)
+        launch_substep_t<kGeneralBW, kGeneralBH, kGeneralNT, kModeField>(A, s);
     } else if (mode == kModeConst) {
-        launch_substep_t<32, 8, 256, kModeConst>(A, s);
+        launch_substep_t<kGeneralBW, kGeneralBH, kGeneralNT, kModeConst>(A, s);
     } else {
         switch (cfg) {
             case 0: launch_substep_t<32, 8, 256, kModeZero>(A, s); break;

@@ -19,6 +19,12 @@ extern const TileConfig kTileConfigs[];
 extern const int kNumTileConfigs;
 extern const int kDefaultTileConfig;
 extern const int kMarchAutoConfig;
+// Tile of the rotated and per-cell modes (they ignore the configuration): the
+// slope and face phases fit two passes of 512 threads.  Substep with a Coriolis
+// field at 1500^2: 56.1 us against 62 to 64 for 16x16/256, 16x14/256 and
+// 32x7/256; at 640x417 all of them take 11 us, 32x8/256 14.4 and 32x16/256 20.8.
+constexpr int kGeneralBW = 32, kGeneralBH = 14, kGeneralNT = 512;
+constexpr TileConfig kGeneralTile = {kGeneralBW, kGeneralBH, kGeneralNT, "32x14/512"};
 // configurations kFirstMarchConfig .. kNumTileConfigs-1 are column marching
 constexpr int kFirstMarchConfig = 7;
 // configuration used when the caller passes -1
@@ -30,7 +36,7 @@ const char* last_error();
 int check_launch(const char* what);
 int validate_domain(const gocean_domain_t* d);
 void fill_args(const gocean_domain_t* d, SubstepArgs& A);
-// true when one residual correction divides every float by d correctly
+// true when div_k's two instructions divide every float by d correctly
 // rounded (checked once per value of d, on the host)
 bool two_step_exact(float d);
 // the substep's FAST arithmetic is exact for these constants: one-correction
