@@ -77,9 +77,10 @@ int validate_domain(const gocean_domain_t* d) {
 // ---------------------------------------------------------------------------
 // RN(n r + RN(n l)) with r = RN(1/d), l = RN(1/d - r) (div_k) is the correctly
 // rounded n/d for most d but is not guaranteed for all.  Scaling n by a power
-// of two scales every intermediate exactly, so the check over the 2^23
-// significands of n in [1, 2) decides it for every n of normal magnitude (and
-// -n by symmetry).  Done once per divisor value on the host, with the hardware
+// of two scales every intermediate exactly as long as n l stays normal, so the
+// check over the 2^23 significands of n in [1, 2) decides it for quotients down
+// to 2^-101 (and -n by symmetry); below that the last place can differ, as it
+// can with a residual correction, whose residual is subnormal there too.  Done once per divisor value on the host, with the hardware
 // FMA when the CPU has one.
 namespace {
 

@@ -20,9 +20,9 @@ extern const int kNumTileConfigs;
 extern const int kDefaultTileConfig;
 extern const int kMarchAutoConfig;
 // Tile of the rotated and per-cell modes (they ignore the configuration): the
-// slope and face phases fit two passes of 512 threads.  Substep with a Coriolis
-// field at 1500^2: 56.1 us against 62 to 64 for 16x16/256, 16x14/256 and
-// 32x7/256; at 640x417 all of them take 11 us, 32x8/256 14.4 and 32x16/256 20.8.
+// slope and face phases fit two passes of 512 threads.  us per substep with a
+// Coriolis field, one stream, at 640x417 / 1500^2: 11.3 / 57.2 against
+// 11.6 / 61.2 for 16x16/256, 11.0 / 62.4 for 16x14/256, 14.6 / 70.8 for 32x8/256.
 constexpr int kGeneralBW = 32, kGeneralBH = 14, kGeneralNT = 512;
 constexpr TileConfig kGeneralTile = {kGeneralBW, kGeneralBH, kGeneralNT, "32x14/512"};
 // configurations kFirstMarchConfig .. kNumTileConfigs-1 are column marching
