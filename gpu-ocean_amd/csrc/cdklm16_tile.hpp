@@ -38,7 +38,7 @@ constexpr int kPeriodic = 2;
 // registers.
 struct SubstepDerived {
     float vdx, udy, r_two_g, r_dx, r_dy;   // dx/(2g), dy/(2g), 1/(2g), 1/dx, 1/dy
-    float l_two_g, l_dx, l_dy;             // 1/d - RN(1/d), for div_k
+    float l_two_g, l_dx, l_dy;             // low parts of the reciprocals for div_k, set by fast_arith
     float half_g, two_g, theta_g, dxf, dyf;   // 0.5 g, 2 g, theta g, dx f, dy f
     // thresholds of the marching kernel's wave-uniform fast paths: a corner
     // depth in (kDryFlag, plain_hi) is neither land nor the dry flag, and
@@ -84,7 +84,8 @@ struct SubstepArgs : SubstepDerived {
     __host__ __device__ int bc_w() const { return (int)((flags >> 6) & 3u); }
     __host__ __device__ int rk_order() const { return (int)((flags >> 8) & 3u); }
     __host__ __device__ int rk_step() const { return (int)((flags >> 10) & 3u); }
-    // bit 12: divisions by dx, dy and 2g may take one residual correction
+    // bit 12: divisions by dx, dy and 2g may take div_k's two instructions, and
+    // the wet wave speeds the Newton square root
     __host__ __device__ bool fast_arith() const { return (flags >> 12) & 1u; }
     __host__ __device__ void set_fast_arith(bool on) { flags = (flags & ~(1u << 12)) | ((on ? 1u : 0u) << 12); }
     __host__ __device__ void set_flags(int n, int e, int s_, int w, int order, int step) {
@@ -177,9 +178,7 @@ inline SubstepDerived substep_derive(float dx, float dy, float g, float theta, f
     D.r_two_g = 1.0f / D.two_g;
     D.r_dx = 1.0f / dx;
     D.r_dy = 1.0f / dy;
-    D.l_two_g = reciprocal_low(D.two_g);
-    D.l_dx = reciprocal_low(dx);
-    D.l_dy = reciprocal_low(dy);
+    D.l_two_g = D.l_dx = D.l_dy = 0.0f;
     D.plain_hi = (land >= 1.0f) ? 0.5f * land : -INFINITY;
     const float c = 0.50001f * flux_eps;
     D.face_lo = fmaxf(fmaxf(cutoff, 0.0f), (c * c) / g * 1.00001f);
@@ -278,15 +277,14 @@ __device__ __forceinline__ float div_r(float n, float d, float r) {
 }
 
 // n/d for a launch-constant divisor d (dx, dy, 2g): with the reciprocal as an
-// unevaluated sum r + l (r = RN(1/d), l = RN(1/d - r), formed on the host),
+// unevaluated sum r + l (r = RN(1/d), l next to 1/d - r, formed on the host),
 // RN(n r + RN(n l)) in two instructions (Brisebarre, Muller & Raina,
 // "Accelerating correctly rounded floating-point division when the divisor is
-// known in advance", IEEE Trans. Computers 53 (2004); div_r takes five).  It
-// is correctly rounded for most divisors; the host enables it (SubstepArgs
-// fast_arith()) only for divisors for which it has checked every float
-// significand of n (fast_arith_exact in gocean_fwd.hip); otherwise div_r runs.
-// Quotients below 2^-101, where n l is subnormal, can be one unit in the last
-// place off.
+// known in advance", IEEE Trans. Computers 53 (2004); div_r takes five).  The
+// host chooses l and enables the form (SubstepArgs fast_arith()) only for
+// divisors for which it has checked every float significand of n (divisor_low
+// in gocean_fwd.hip); otherwise div_r runs.  Quotients below 2^-126 r / |l|,
+// where n l is subnormal, can be one unit in the last place off.
 template <bool FAST>
 __device__ __forceinline__ float div_k(float n, float d, float r, float l) {
     if constexpr (FAST) return fmaf(n, r, n * l);
@@ -313,7 +311,7 @@ __device__ __forceinline__ float sqrt_rn(float x) {
 // normal range they differ.  Five instructions against sqrt_rn's nine.  The
 // kernels take it (FAST) only where the argument is g h with h above the
 // depth cutoff, and the host enables FAST only when RN(g cutoff) >= 2^-60
-// (fast_arith_exact in gocean_fwd.hip).
+// (fast_arith in gocean_fwd.hip).
 __device__ __forceinline__ float sqrt_newton(float x) {
     const float y = __builtin_amdgcn_rsqf(x);
     const float g = x * y;

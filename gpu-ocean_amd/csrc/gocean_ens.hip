@@ -456,7 +456,7 @@ struct gocean_ensemble {
     int bw = 32, bh = 16, nt = 256;
     int n_tiles = 0;
     int device = 0;
-    bool fast_arith = false;   // fast_arith_exact holds for every member
+    bool fast_arith = false;   // fast_arith holds for every member
     float friction = 0.0f;     // largest r of the members
     bool fits = true;          // every member's planes suit the marching kernel's 32-bit offsets
     EnsMember* d_members = nullptr;
@@ -622,7 +622,8 @@ int gocean_ensemble_create(const gocean_member_t* members, int n, int tile_confi
     E->friction = 0.0f;
     for (int k = 0; k < n; ++k) {
         const gocean_domain_t& d = members[k].domain;
-        E->fast_arith = E->fast_arith && fast_arith_exact(d.g, d.dx, d.dy, d.depth_cutoff);
+        SubstepDerived D;
+        E->fast_arith = fast_arith(d.g, d.dx, d.dy, d.depth_cutoff, D) && E->fast_arith;
         E->friction = std::max(E->friction, d.r);
     }
     const TileConfig& tc = (E->mode == kModeZero) ? kTileConfigs[E->cfg] : kGeneralTile;
@@ -658,6 +659,7 @@ int gocean_ensemble_create(const gocean_member_t* members, int n, int tile_confi
         M.bc_n = d.bc_north; M.bc_e = d.bc_east; M.bc_s = d.bc_south; M.bc_w = d.bc_west;
         static_cast<SubstepDerived&>(M) =
             substep_derive(d.dx, d.dy, d.g, d.theta, d.f, d.flux_slope_eps, d.depth_cutoff, d.land_value);
+        (void)fast_arith(d.g, d.dx, d.dy, d.depth_cutoff, M);
         if (m.state_offset < 0 || m.hi_offset < 0 || m.hm_offset < 0) {
             delete E;
             return set_error(GOCEAN_EINVAL, "member %d: negative buffer offset", k);

@@ -75,17 +75,22 @@ int validate_domain(const gocean_domain_t* d) {
 // ---------------------------------------------------------------------------
 // division by a launch constant in two instructions
 // ---------------------------------------------------------------------------
-// RN(n r + RN(n l)) with r = RN(1/d), l = RN(1/d - r) (div_k) is the correctly
-// rounded n/d for most d but is not guaranteed for all.  Scaling n by a power
-// of two scales every intermediate exactly as long as n l stays normal, so the
-// check over the 2^23 significands of n in [1, 2) decides it for quotients down
-// to 2^-101 (and -n by symmetry); below that the last place can differ, as it
-// can with a residual correction, whose residual is subnormal there too.  Done once per divisor value on the host, with the hardware
-// FMA when the CPU has one.
+// RN(n r + RN(n l)) with r = RN(1/d) and l next to 1/d - r (div_k) is the
+// correctly rounded n/d for nearly every d when l is RN(1/d - r), and not for
+// the rest: there some quotients lie so close to the middle of two floats that
+// the rounding of l decides, and one of l's two neighbours serves.  Of 3000
+// random significands 41 fail with RN(1/d - r) (1000/3 is one), 2 with all
+// three.  Scaling n by a power of two scales every intermediate exactly while
+// n l stays normal, so a scan over the 2^23 significands of n in [1, 2) decides
+// it for quotients down to 2^-126 r / |l| (about 2^-101 for d = 300, 2^-92 for
+// 19.62; -n by symmetry).  Below that n l is rounded to a multiple of 2^-149,
+// and the quotient can be one unit in the last place off, as div_r's can below
+// about 2^-103 / d, where its residuals are subnormal.
+// Done once per divisor value on the host (10 ms), with the hardware FMA when
+// the CPU has one.
 namespace {
 
-__attribute__((target("fma"))) bool two_step_scan_fma(float d) {
-    const float r = 1.0f / d, l = reciprocal_low(d);
+__attribute__((target("fma"))) bool two_step_scan_fma(float d, float r, float l) {
     for (uint32_t m = 0; m < (1u << 23); ++m) {
         uint32_t bits = 0x3f800000u | m;
         float n;
@@ -95,8 +100,7 @@ __attribute__((target("fma"))) bool two_step_scan_fma(float d) {
     return true;
 }
 
-bool two_step_scan_libm(float d) {
-    const float r = 1.0f / d, l = reciprocal_low(d);
+bool two_step_scan_libm(float d, float r, float l) {
     for (uint32_t m = 0; m < (1u << 23); ++m) {
         uint32_t bits = 0x3f800000u | m;
         float n;
@@ -107,31 +111,43 @@ bool two_step_scan_libm(float d) {
 }
 
 std::mutex g_div_mu;
-std::unordered_map<uint32_t, bool> g_div_ok;
+std::unordered_map<uint32_t, DivisorLow> g_div;
 
 }  // namespace
 
-bool two_step_exact(float d) {
-    if (!(d > 0.0f) || !std::isnormal(d) || !std::isnormal(1.0f / d)) return false;
+DivisorLow divisor_low(float d) {
+    if (!(d > 0.0f) || !std::isnormal(d) || !std::isnormal(1.0f / d)) return DivisorLow{0.0f, false};
     uint32_t key;
     std::memcpy(&key, &d, 4);
     {
         std::lock_guard<std::mutex> lock(g_div_mu);
-        auto it = g_div_ok.find(key);
-        if (it != g_div_ok.end()) return it->second;
+        auto it = g_div.find(key);
+        if (it != g_div.end()) return it->second;
     }
-    const bool ok = __builtin_cpu_supports("fma") ? two_step_scan_fma(d) : two_step_scan_libm(d);
+    const float r = 1.0f / d, l = reciprocal_low(d);
+    const bool fma = __builtin_cpu_supports("fma");
+    DivisorLow best{l, false};
+    for (const float c : {l, std::nextafter(l, INFINITY), std::nextafter(l, -INFINITY)}) {
+        if (fma ? two_step_scan_fma(d, r, c) : two_step_scan_libm(d, r, c)) {
+            best = DivisorLow{c, true};
+            break;
+        }
+    }
     std::lock_guard<std::mutex> lock(g_div_mu);
-    g_div_ok[key] = ok;
-    return ok;
+    g_div[key] = best;
+    return best;
 }
 
-bool fast_arith_exact(float g, float dx, float dy, float cutoff) {
+bool fast_arith(float g, float dx, float dy, float cutoff, SubstepDerived& D) {
     // sqrt_newton equals sqrt_rn for arguments >= 2^-60; the wave speeds take
     // it only for depths above the cutoff, whose g h rounds to >= RN(g cutoff)
     const float lo = g * cutoff;
     if (!(g > 0.0f) || !std::isfinite(g) || !(lo >= 0x1p-60f)) return false;
-    return two_step_exact(2.0f * g) && two_step_exact(dx) && two_step_exact(dy);
+    const DivisorLow two_g = divisor_low(2.0f * g), x = divisor_low(dx), y = divisor_low(dy);
+    D.l_two_g = two_g.low;
+    D.l_dx = x.low;
+    D.l_dy = y.low;
+    return two_g.exact && x.exact && y.exact;
 }
 
 void fill_args(const gocean_domain_t* d, SubstepArgs& A) {
@@ -144,7 +160,7 @@ void fill_args(const gocean_domain_t* d, SubstepArgs& A) {
     A.set_flags(d->bc_north, d->bc_east, d->bc_south, d->bc_west, d->rk_order, 0);
     static_cast<SubstepDerived&>(A) =
         substep_derive(A.dx, A.dy, A.g, A.theta, A.f, A.flux_eps, A.cutoff, A.land);
-    A.set_fast_arith(fast_arith_exact(A.g, A.dx, A.dy, A.cutoff));
+    A.set_fast_arith(fast_arith(A.g, A.dx, A.dy, A.cutoff, A));
 }
 
 // ---------------------------------------------------------------------------
@@ -683,6 +699,15 @@ int gocean_adjoint_set_record_tile_config(int cfg) {
 int gocean_adjoint_record_tile_config(void) { return g_record_cfg; }
 
 int gocean_default_tile_config(int, int) { return default_tile_config(); }
+
+int gocean_division_constants(float d, float* high, float* low) {
+    clear_error();
+    if (!high || !low) return set_error(GOCEAN_EINVAL, "NULL pointer");
+    const DivisorLow q = divisor_low(d);
+    *high = 1.0f / d;
+    *low = q.low;
+    return q.exact ? 1 : 0;
+}
 
 int gocean_sqrt_newton_check(uint32_t lo_bits, uint32_t hi_bits, unsigned long long* mismatches) {
     clear_error();

@@ -36,13 +36,18 @@ const char* last_error();
 int check_launch(const char* what);
 int validate_domain(const gocean_domain_t* d);
 void fill_args(const gocean_domain_t* d, SubstepArgs& A);
-// true when div_k's two instructions divide every float by d correctly
-// rounded (checked once per value of d, on the host)
-bool two_step_exact(float d);
-// the substep's FAST arithmetic is exact for these constants: one-correction
-// division by dx, dy and 2g, and the Newton square root of g h for h above
-// the depth cutoff
-bool fast_arith_exact(float g, float dx, float dy, float cutoff);
+// the low part l of div_k's reciprocal r + l of a divisor d, and whether the two
+// instructions then divide every float by d correctly rounded (searched and
+// checked once per value of d, on the host)
+struct DivisorLow {
+    float low;
+    bool exact;
+};
+DivisorLow divisor_low(float d);
+// the substep's FAST arithmetic is exact for these constants: two-instruction
+// division by dx, dy and 2g, whose low parts it writes to D, and the Newton
+// square root of g h for h above the depth cutoff
+bool fast_arith(float g, float dx, float dy, float cutoff, SubstepDerived& D);
 // the column-marching kernels' 32-bit plane offsets cover a domain of this
 // height and pitches
 bool march_fits(int ny, int pitch, int hi_pitch);

@@ -194,6 +194,13 @@ int gocean_tile_configs(const char** names, int max);
  * take a 2-D tile instead). */
 int gocean_default_tile_config(int nx, int ny);
 
+/* The constants of the substep kernels' two-instruction division by d (the cell
+ * sizes and 2g): n/d = RN(n high + RN(n low)).  Returns 1 when the host has
+ * found this correctly rounded for every float significand of n, 0 when the
+ * kernels use the generic correctly rounded division instead, and a negative
+ * error code for a NULL pointer.  No counterpart in the reference. */
+int gocean_division_constants(float d, float* high, float* low);
+
 /* Device self-check of the square root the substep kernels take for wave
  * speeds when the host enables their fast arithmetic: counts the float bit
  * patterns in [lo_bits, hi_bits] (positive floats, lo_bits <= hi_bits <=
