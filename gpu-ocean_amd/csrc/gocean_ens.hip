@@ -458,6 +458,7 @@ struct gocean_ensemble {
     int device = 0;
     bool fast_arith = false;   // fast_arith holds for every member
     float friction = 0.0f;     // largest r of the members
+    int general = 0;           // tile of the rotated and per-cell modes (kGeneralTiles)
     bool fits = true;          // every member's planes suit the marching kernel's 32-bit offsets
     EnsMember* d_members = nullptr;
     int* d_tile_member = nullptr;
@@ -484,6 +485,15 @@ namespace gocean {
 template <int BW, int BH, int NT, int MODE>
 static void ens_launch_t(const EnsLaunch& L, hipStream_t s) {
     hipLaunchKernelGGL((k_ens_substep<BW, BH, NT, MODE>), dim3(L.n_tiles), dim3(NT), 0, s, L);
+}
+
+template <int MODE>
+static void ens_general(int tile, const EnsLaunch& L, hipStream_t s) {
+    switch (tile) {
+        case 0: ens_launch_t<32, 14, 512, MODE>(L, s); break;
+        case 1: ens_launch_t<16, 16, 256, MODE>(L, s); break;
+        default: ens_launch_t<32, 8, 256, MODE>(L, s); break;
+    }
 }
 
 using EnsKernel = void (*)(EnsLaunch);
@@ -521,9 +531,9 @@ static int ens_launch(const gocean_ensemble* E, EnsLaunch L, hipStream_t s) {
     L.tile_member = E->d_tile_member;
     L.n_tiles = E->n_tiles;
     if (E->mode == kModeField) {
-        ens_launch_t<kGeneralBW, kGeneralBH, kGeneralNT, kModeField>(L, s);
+        ens_general<kModeField>(E->general, L, s);
     } else if (E->mode == kModeConst) {
-        ens_launch_t<kGeneralBW, kGeneralBH, kGeneralNT, kModeConst>(L, s);
+        ens_general<kModeConst>(E->general, L, s);
     } else {
         switch (E->cfg) {
             case 0: ens_launch_t<32, 8, 256, kModeZero>(L, s); break;
@@ -626,7 +636,12 @@ int gocean_ensemble_create(const gocean_member_t* members, int n, int tile_confi
         E->fast_arith = fast_arith(d.g, d.dx, d.dy, d.depth_cutoff, D) && E->fast_arith;
         E->friction = std::max(E->friction, d.r);
     }
-    const TileConfig& tc = (E->mode == kModeZero) ? kTileConfigs[E->cfg] : kGeneralTile;
+    if (E->mode != kModeZero) {
+        std::vector<int> nx(n), ny(n);
+        for (int k = 0; k < n; ++k) { nx[k] = members[k].domain.nx; ny[k] = members[k].domain.ny; }
+        E->general = general_tile(E->mode, nx.data(), ny.data(), n);
+    }
+    const TileConfig& tc = (E->mode == kModeZero) ? kTileConfigs[E->cfg] : kGeneralTiles[E->general];
     E->bw = tc.bw; E->bh = tc.bh; E->nt = tc.nt;
     if (E->bh == 0) {
         std::vector<EnsMember> shape(n);
@@ -699,7 +714,7 @@ int gocean_ensemble_set_tile_config(gocean_ensemble_t* E, int tile_config) {
     // work already queued may still read the old tables
     if (hipDeviceSynchronize() != hipSuccess) return check_launch("ensemble tile configuration");
     E->cfg = tile_config;
-    const TileConfig& tc = (E->mode == kModeZero) ? kTileConfigs[E->cfg] : kGeneralTile;
+    const TileConfig& tc = (E->mode == kModeZero) ? kTileConfigs[E->cfg] : kGeneralTiles[E->general];
     E->bw = tc.bw; E->bh = tc.bh; E->nt = tc.nt;
     if (E->bh == 0) E->bh = ens_march_rows(E->members, E->fast_arith);
     std::vector<int> tile_member;

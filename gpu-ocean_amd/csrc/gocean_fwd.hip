@@ -210,6 +210,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WGRID ? 4 :
     march::march_strip<FAST, WGRID, STAGE>(A, sx, sy, A.march_bh);
 }
 
+static int compute_units() {
+    int dev = 0, cus = 256;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+        (void)hipGetLastError();
+        cus = 256;
+    }
+    return cus;
+}
+
 // waves of a kernel that the device holds at once: 4 SIMDs per CU, each
 // holding as many waves as its 512 vector registers per lane allow
 int resident_waves(const void* kernel) {
@@ -217,14 +226,9 @@ int resident_waves(const void* kernel) {
     hipFuncAttributes fa;
     if (hipFuncGetAttributes(&fa, kernel) == hipSuccess && fa.numRegs > 0) regs = fa.numRegs;
     else (void)hipGetLastError();
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
-        (void)hipGetLastError();
-        cus = 256;
-    }
     const int alloc = (regs + 7) / 8 * 8;
     const int per_simd = std::max(1, std::min(8, 512 / alloc));
-    return cus * 4 * per_simd;
+    return compute_units() * 4 * per_simd;
 }
 
 // Rows per strip for a column-marching kernel over domains of the given
@@ -316,6 +320,45 @@ static void launch_substep_t(SubstepArgs A, hipStream_t s) {
     A.tiles_y = (A.ny + BH - 1) / BH;
     const int nb = A.tiles_x * A.tiles_y;
     hipLaunchKernelGGL((k_substep<BW, BH, NT, MODE>), dim3(nb), dim3(NT), 0, s, A);
+}
+
+// The tile of least cost, the tiles that the fullest CU takes times a tile's
+// time relative to 32x14/512.  32x14 makes the least halo per cell and its slope
+// and face phases fit two passes of 512 threads; the smaller tiles waste less
+// on domains of few rows or columns and spread a few hundred tiles more evenly.
+// Where every CU has at most one 32x14 tile the time is a tile's own, and its
+// 512 threads are the fastest; where the costs are level it stays (400^2 and
+// 256 members of 24^2 are within 3 % either way).  ns per tile at 2048^2 (32x14, 16x16, 32x8):
+// constant rotation 8.3, 5.3, 5.3; fields with one north vector 10.6, 6.6, 7.7,
+// with varying ones 11.6, 7.7, 8.8.  us per substep, 32x14 / 16x16 / 32x8:
+// rotated 512^2 11.2 / 10.0 / 10.2, 1500^2 45.4 / 50.0 / 50.0, 1024 members of
+// 16^2 24.6 / 11.1 / 18.1; fields 512^2 13.1 / 12.4 / 12.3, 96x80 8.4 / 9.5 /
+// 9.3, 1500^2 62.3 / 70.7 / 80.0, 1024 members of 16^2 29.6 / 13.5 / 22.9.
+int general_tile(int mode, const int* nx, const int* ny, int n) {
+    constexpr double cost[2][3] = {{1.0, 0.65, 0.65}, {1.0, 0.70, 0.75}};
+    static std::atomic<int> known{0};
+    if (!known.load()) known.store(compute_units());
+    const int cus = known.load();
+    int best = 0;
+    double least = 0.0;
+    for (int k = 0; k < 3; ++k) {
+        const TileConfig& t = kGeneralTiles[k];
+        long long tiles = 0;
+        for (int m = 0; m < n; ++m) tiles += (long long)((nx[m] + t.bw - 1) / t.bw) * ((ny[m] + t.bh - 1) / t.bh);
+        if (k == 0 && tiles <= cus) return 0;
+        const double c = (double)((tiles + cus - 1) / cus) * cost[mode == kModeField][k] - (k == 0 ? 0.1 : 0.0);
+        if (k == 0 || c < least) { least = c; best = k; }
+    }
+    return best;
+}
+
+template <int MODE>
+static void launch_general(const SubstepArgs& A, hipStream_t s) {
+    switch (general_tile(MODE, &A.nx, &A.ny, 1)) {
+        case 0: launch_substep_t<32, 14, 512, MODE>(A, s); break;
+        case 1: launch_substep_t<16, 16, 256, MODE>(A, s); break;
+        default: launch_substep_t<32, 8, 256, MODE>(A, s); break;
+    }
 }
 
 // recording variant (zero rotation only): also writes the branch record
@@ -419,11 +462,10 @@ int launch_substep(const SubstepArgs& A, int cfg, bool field, hipStream_t s) {
         return set_error(GOCEAN_EINVAL, "tile configuration %d (column marching) needs planes below 4 GiB", cfg);
     const int mode = substep_mode(A, field);
     if (mode == kModeField) {
-        // per-cell Coriolis / north fields, and rotated grids below: one
-        // general configuration (kGeneralBW)
-        launch_substep_t<kGeneralBW, kGeneralBH, kGeneralNT, kModeField>(A, s);
+        // per-cell Coriolis / north fields, and rotated grids below
+        launch_general<kModeField>(A, s);
     } else if (mode == kModeConst) {
-        launch_substep_t<kGeneralBW, kGeneralBH, kGeneralNT, kModeConst>(A, s);
+        launch_general<kModeConst>(A, s);
     } else {
         switch (cfg) {
             case 0: launch_substep_t<32, 8, 256, kModeZero>(A, s); break;

@@ -19,12 +19,10 @@ extern const TileConfig kTileConfigs[];
 extern const int kNumTileConfigs;
 extern const int kDefaultTileConfig;
 extern const int kMarchAutoConfig;
-// Tile of the rotated and per-cell modes (they ignore the configuration): the
-// slope and face phases fit two passes of 512 threads.  us per substep with a
-// Coriolis field, one stream, at 640x417 / 1500^2: 11.3 / 57.2 against
-// 11.6 / 61.2 for 16x16/256, 11.0 / 62.4 for 16x14/256, 14.6 / 70.8 for 32x8/256.
-constexpr int kGeneralBW = 32, kGeneralBH = 14, kGeneralNT = 512;
-constexpr TileConfig kGeneralTile = {kGeneralBW, kGeneralBH, kGeneralNT, "32x14/512"};
+// Tiles of the rotated and per-cell modes (they ignore the configuration), and
+// the choice among them for a mode and n domains
+constexpr TileConfig kGeneralTiles[] = {{32, 14, 512, "32x14/512"}, {16, 16, 256, "16x16/256"}, {32, 8, 256, "32x8/256"}};
+int general_tile(int mode, const int* nx, const int* ny, int n);
 // configurations kFirstMarchConfig .. kNumTileConfigs-1 are column marching
 constexpr int kFirstMarchConfig = 7;
 // configuration used when the caller passes -1

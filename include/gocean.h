@@ -246,8 +246,8 @@ int gocean_ensemble_destroy(gocean_ensemble_t* ens);
 /* Switch the tile configuration of the batched substep (index into
  * gocean_tile_configs; -1 = default) and rebuild the tile -> member map, for
  * an autotuner.  Synchronises the device first and drops a captured graph
- * (capture again).  Members with per-cell fields or a rotated grid always use
- * the 32x8 tile. */
+ * (capture again).  Members with per-cell fields or a rotated grid use a 2-D
+ * tile chosen from their sizes, whatever the configuration. */
 int gocean_ensemble_set_tile_config(gocean_ensemble_t* ens, int tile_config);
 /* n_members, total tiles and kernel mode (0 zero angle, 1 constant north,
  * 2 per-cell fields). */
