@@ -37,6 +37,7 @@ struct EnsMember : SubstepDerived {
     long long work_off;
     int ftiles_x, ftile_begin, atiles_x, atile_begin;
     int astrips_x, astrip_begin;   // the member's strips in the column-marching reverse launch
+    int rstrips_x, rstrip_begin;   // and in the column-marching recording launch
     float Dx, Dy, Ddx, Ddy, g_dx, g_dy;   // as AdjTileArgs
 };
 
@@ -297,7 +298,7 @@ __global__ __launch_bounds__(kEnsTapeNT) __attribute__((amdgpu_waves_per_eu(8)))
 }
 
 // column-marching recording substep over every member's strips (the strip
-// map of the ensemble's marching configuration)
+// map of the adjoint setup)
 template <bool FAST>
 __global__ __launch_bounds__(256) void k_ens_march_tape(EnsTapeLaunch L, int bh, int n_strips) {
     const int wave = xcd_band(blockIdx.x, gridDim.x) * 4 + march::wave_in_group();
@@ -327,9 +328,9 @@ __global__ __launch_bounds__(256) void k_ens_march_tape(EnsTapeLaunch L, int bh,
     A.dt = 0.0f;
     A.set_flags(M.bc_n, M.bc_e, M.bc_s, M.bc_w, 2, L.rk_step);
     static_cast<SubstepDerived&>(A) = M;
-    A.tiles_x = M.tiles_x; A.tiles_y = 0;
-    const int lt = wave - M.tile_begin;
-    const int sy = lt / M.tiles_x, sx = lt - sy * M.tiles_x;
+    A.tiles_x = M.rstrips_x; A.tiles_y = 0;
+    const int lt = wave - M.rstrip_begin;
+    const int sy = lt / M.rstrips_x, sx = lt - sy * M.rstrips_x;
     march::march_strip<FAST, false, march::kStageAny, true>(A, sx, sy, bh);
 }
 
@@ -452,6 +453,7 @@ struct gocean_ensemble {
     int n = 0;
     int rk_order = 2;
     int cfg = 1;
+    bool default_cfg = true;   // cfg is the default's choice, not the caller's
     int mode = kModeZero;
     int bw = 32, bh = 16, nt = 256;
     int n_tiles = 0;
@@ -476,6 +478,10 @@ struct gocean_ensemble {
     // every member's planes fit its 32-bit offsets
     int* d_astrip_member = nullptr;
     int n_astrips = 0, adj_bh = 0;
+    // and of the column-marching recording launch
+    int* d_rstrip_member = nullptr;
+    int n_rstrips = 0, rec_bh = 0;
+    bool rec_march = true;     // the default configuration records through it
     long long adj_cells = 0;
     bool adj_march_fits = false;
 };
@@ -524,6 +530,20 @@ static int ens_march_rows(const std::vector<EnsMember>& members, bool fast_arith
     const int resident = resident_waves((const void*)(fast_arith ? ens_march_kernel<true>(march::kStageSecond)
                                                                  : ens_march_kernel<false>(march::kStageSecond)));
     return march_rows(strips.data(), ny.data(), (int)members.size(), resident, 1);
+}
+
+// Estimated us of a column-marching launch: each wave's rows and prologue, in
+// rounds of the waves resident; a round that leaves CUs short of workgroups is
+// faster by `idle` for each one missing.  The constants of a kernel are fitted
+// to launches of 16 to 4096 members of 8x8 to 200x133 cells.
+static double strips_us(const std::vector<int>& strips, const std::vector<int>& ny, int rows, int resident,
+                        double row_us, double prologue, double idle) {
+    long long waves = 0;
+    for (size_t k = 0; k < strips.size(); ++k) waves += (long long)strips[k] * ((ny[k] + rows - 1) / rows);
+    const int group = 4 * compute_units(), full = resident / group;
+    const long long rounds = (waves + resident - 1) / resident;
+    const int groups = rounds > 1 ? full : std::min(full, (int)((waves + group - 1) / group));
+    return row_us * (rows + prologue) * (double)rounds * (1.0 - idle * (full - groups));
 }
 
 static int ens_launch(const gocean_ensemble* E, EnsLaunch L, hipStream_t s) {
@@ -596,6 +616,7 @@ int gocean_ensemble_create(const gocean_member_t* members, int n, int tile_confi
     E->n = n;
     E->rk_order = members[0].domain.rk_order;
     E->cfg = tile_config < 0 ? default_tile_config() : tile_config;
+    E->default_cfg = tile_config < 0;
     bool any_field = false, any_const = false;
     for (int k = 0; k < n; ++k) {
         const gocean_domain_t& d = members[k].domain;
@@ -710,6 +731,7 @@ int gocean_ensemble_set_tile_config(gocean_ensemble_t* E, int tile_config) {
     if (tile_config >= kFirstMarchConfig && !E->fits)
         return set_error(GOCEAN_EINVAL, "tile configuration %d (column marching) needs member planes below 4 GiB",
                          tile_config);
+    E->default_cfg = tile_config < 0;
     if (tile_config < 0) tile_config = E->fits ? default_tile_config() : kDefaultTileConfig;
     // work already queued may still read the old tables
     if (hipDeviceSynchronize() != hipSuccess) return check_launch("ensemble tile configuration");
@@ -754,6 +776,7 @@ int gocean_ensemble_destroy(gocean_ensemble_t* E) {
     (void)hipFree(E->d_ftile_member);
     (void)hipFree(E->d_atile_member);
     (void)hipFree(E->d_astrip_member);
+    (void)hipFree(E->d_rstrip_member);
     delete E;
     return 0;
 }
@@ -905,27 +928,57 @@ long long gocean_ensemble_adjoint_setup(gocean_ensemble_t* E, int max_steps) {
     static int resident = 0;
     if (!resident) resident = resident_waves((const void*)k_ens_adj_march);
     const int abh = march_rows(snx.data(), sny.data(), E->n, resident, 8);
+    // column-marching recording launch: rows for whole rounds of its own
+    // resident waves, four per SIMD where the plain forward kernel has five
+    // (in the forward's strips 256 members of 64^2 took two rounds: 43 us per
+    // substep, 38 in these)
+    std::vector<int> rnx(E->n), rny(E->n), rstrips;
+    for (int k = 0; k < E->n; ++k) {
+        rnx[k] = (E->members[k].nx + march::kOut - 1) / march::kOut;
+        rny[k] = E->members[k].ny;
+    }
+    const int rec_resident = resident_waves(E->fast_arith ? (const void*)k_ens_march_tape<true>
+                                                          : (const void*)k_ens_march_tape<false>);
+    const int rbh = march_rows(rnx.data(), rny.data(), E->n, rec_resident, 1);
+    // 32x16 tiles instead, 4 us for each that a CU takes, where a few per CU
+    // beat the strips' rows: us per substep, strips / tiles, 700 members of
+    // 20x32 34.1 / 30.9, of 24x64 54.8 / 49.6, 1024 of 16^2 25.2 / 23.8; 1024 of
+    // 64^2 132 / 139, 16 of 512^2 84 / 112.  Other ensembles are within 4 % of
+    // the faster one; past 24 a CU the strips are.
+    const int cus = compute_units();
+    const long long per_cu = ((long long)ftiles.size() + cus - 1) / cus;
+    E->rec_march = !(per_cu > 1 && per_cu <= 24 &&
+                     6.5 + 4.0 * (double)per_cu < strips_us(rnx, rny, rbh, rec_resident, 3.9, 2.0, 0.1));
     for (int k = 0; k < E->n; ++k) {
         EnsMember& M = E->members[k];
         M.astrips_x = snx[k];
         M.astrip_begin = (int)astrips.size();
         for (int t = 0; t < snx[k] * ((sny[k] + abh - 1) / abh); ++t) astrips.push_back(k);
+        M.rstrips_x = rnx[k];
+        M.rstrip_begin = (int)rstrips.size();
+        for (int t = 0; t < rnx[k] * ((rny[k] + rbh - 1) / rbh); ++t) rstrips.push_back(k);
     }
     (void)hipFree(E->d_ftile_member);
     (void)hipFree(E->d_atile_member);
     (void)hipFree(E->d_astrip_member);
+    (void)hipFree(E->d_rstrip_member);
+    E->d_rstrip_member = nullptr;
     E->d_ftile_member = nullptr;
     E->d_atile_member = nullptr;
     E->d_astrip_member = nullptr;
     if (hipMalloc(&E->d_ftile_member, sizeof(int) * ftiles.size()) != hipSuccess ||
         hipMalloc(&E->d_atile_member, sizeof(int) * atiles.size()) != hipSuccess ||
-        hipMalloc(&E->d_astrip_member, sizeof(int) * astrips.size()) != hipSuccess) {
+        hipMalloc(&E->d_astrip_member, sizeof(int) * astrips.size()) != hipSuccess ||
+        hipMalloc(&E->d_rstrip_member, sizeof(int) * rstrips.size()) != hipSuccess) {
         (void)hipGetLastError();
         return set_error(GOCEAN_ENOMEM, "device allocation of the adjoint tile maps failed");
     }
     (void)hipMemcpy(E->d_ftile_member, ftiles.data(), sizeof(int) * ftiles.size(), hipMemcpyHostToDevice);
     (void)hipMemcpy(E->d_atile_member, atiles.data(), sizeof(int) * atiles.size(), hipMemcpyHostToDevice);
     (void)hipMemcpy(E->d_astrip_member, astrips.data(), sizeof(int) * astrips.size(), hipMemcpyHostToDevice);
+    (void)hipMemcpy(E->d_rstrip_member, rstrips.data(), sizeof(int) * rstrips.size(), hipMemcpyHostToDevice);
+    E->n_rstrips = (int)rstrips.size();
+    E->rec_bh = rbh;
     E->n_astrips = (int)astrips.size();
     E->adj_bh = abh;
     E->adj_cells = cells;
@@ -963,12 +1016,11 @@ struct EnsSegment {
         EnsTapeLaunch L;
         L.members = E->d_members; L.tile_member = E->d_ftile_member;
         L.in = in; L.qn = qn; L.out = out; L.tape = tape; L.Hi = Hi; L.dt = dt; L.rk_step = rk_step;
-        if (E->cfg >= kFirstMarchConfig && E->mode == kModeZero) {
-            // the ensemble's marching configuration records through its strips
-            L.tile_member = E->d_tile_member;
-            const dim3 grid((E->n_tiles + 3) / 4), block(256);
-            if (E->fast_arith) hipLaunchKernelGGL((k_ens_march_tape<true>), grid, block, 0, s, L, E->bh, E->n_tiles);
-            else hipLaunchKernelGGL((k_ens_march_tape<false>), grid, block, 0, s, L, E->bh, E->n_tiles);
+        if (E->cfg >= kFirstMarchConfig && E->mode == kModeZero && (E->rec_march || !E->default_cfg)) {
+            L.tile_member = E->d_rstrip_member;
+            const dim3 grid((E->n_rstrips + 3) / 4), block(256);
+            if (E->fast_arith) hipLaunchKernelGGL((k_ens_march_tape<true>), grid, block, 0, s, L, E->rec_bh, E->n_rstrips);
+            else hipLaunchKernelGGL((k_ens_march_tape<false>), grid, block, 0, s, L, E->rec_bh, E->n_rstrips);
         } else {
             hipLaunchKernelGGL(k_ens_substep_tape, dim3(E->n_ftiles), dim3(kEnsTapeNT), 0, s, L);
         }

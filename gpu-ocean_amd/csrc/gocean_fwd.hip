@@ -210,7 +210,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WGRID ? 4 :
     march::march_strip<FAST, WGRID, STAGE>(A, sx, sy, A.march_bh);
 }
 
-static int compute_units() {
+int compute_units() {
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
         (void)hipGetLastError();

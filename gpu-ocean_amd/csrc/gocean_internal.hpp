@@ -51,6 +51,7 @@ bool fast_arith(float g, float dx, float dy, float cutoff, SubstepDerived& D);
 bool march_fits(int ny, int pitch, int hi_pitch);
 // column-marching launch shape: waves the device holds at once for a kernel,
 // and the rows per strip that fill whole rounds of them
+int compute_units();
 int resident_waves(const void* kernel);
 int march_stage(int rk_order, int rk_step, float r);
 int march_rows(const int* strips, const int* ny, int n, int resident, int least);

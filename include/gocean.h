@@ -168,8 +168,9 @@ int gocean_max_dt_static(const gocean_domain_t* d, const float* eta, const float
  * recording forward substep the adjoint entry points run
  * (gocean_adjoint_record / _segment).  Process-wide; every configuration
  * writes the same record.  An ensemble records with its own configuration
- * (gocean_ensemble_set_tile_config): through its strips when that is a
- * column-marching one, else with 32x16/512 tiles.  No counterpart in the
+ * (gocean_ensemble_set_tile_config): through strips of its recording kernel's
+ * own height when that is a column-marching one, else with 32x16/512 tiles; with
+ * the default, whichever suits its members' sizes.  No counterpart in the
  * reference (the adjoint is new); it lets a tuner pick the fastest recording
  * tile, as for the forward. */
 int gocean_adjoint_set_record_tile_config(int cfg);

@@ -218,3 +218,27 @@ def test_ensemble_marching_record_equals_tile_record(keep):
         if not H.normal_equal(ga, gb):
             raise AssertionError(f"tile {tile}: gradients differ at {int(np.sum(ga != gb))} entries, first "
                                  f"{H.diff_report(ga, gb, 8)}")
+
+
+@pytest.mark.parametrize("n,size", [(700, (16, 16)), (300, (20, 33)), (40, (20, 12)), (3, (130, 70))])
+def test_default_ensemble_record_follows_the_sizes(n, size):
+    """The default configuration records through tiles (the first two) or
+    strips of the recording kernel's own height: the same bits as the explicit
+    configurations, also when the configuration changes after the setup."""
+    from SWESimulators import CDKLM16Ensemble
+    from test_gpu_ensemble import members
+    _say("default ensemble record", n, size)
+    Common, G, A = _mods()
+    ms = members(seed=11, sizes=(size,) * n)
+    ref = _ens_run(ms, 1, 3, 3, True, 4)
+    for tile in (None, 9):
+        got = _ens_run(ms, tile, 3, 3, True, 4)
+        assert np.array_equal(ref[0], got[0]) and H.normal_equal(ref[1], got[1]), tile
+    ens = CDKLM16Ensemble.CDKLM16Ensemble(Common.HIPContext(0), ms, rk_order=2, courant_number=0.6)
+    state0 = ens.state[0].clone()
+    ea = A.EnsembleAdjoint(ens, checkpoint_every=3, keep_records=True)
+    for tile in (-1, 7, 1, 9):
+        ens.set_tile_config(tile)
+        out = ea.forward(state0, 3)
+        torch.cuda.synchronize()
+        assert np.array_equal(ref[0], out.cpu().numpy()), tile
