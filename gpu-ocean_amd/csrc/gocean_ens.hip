@@ -518,20 +518,6 @@ static void ens_march(EnsLaunch L, int bh, bool fast_arith, float r, hipStream_t
                        dim3((L.n_tiles + 3) / 4), dim3(256), 0, s, L);
 }
 
-// rows per strip of the ensemble's column-marching launch (configuration
-// with bh == 0): whole rounds of resident waves over all members' strips
-static int ens_march_rows(const std::vector<EnsMember>& members, bool fast_arith) {
-    std::vector<int> strips, ny;
-    for (const EnsMember& M : members) {
-        strips.push_back((M.nx + march::kOut - 1) / march::kOut);
-        ny.push_back(M.ny);
-    }
-    // the second stage is the larger kernel of the two
-    const int resident = resident_waves((const void*)(fast_arith ? ens_march_kernel<true>(march::kStageSecond)
-                                                                 : ens_march_kernel<false>(march::kStageSecond)));
-    return march_rows(strips.data(), ny.data(), (int)members.size(), resident, 1);
-}
-
 // Estimated us of a column-marching launch: each wave's rows and prologue, in
 // rounds of the waves resident; a round that leaves CUs short of workgroups is
 // faster by `idle` for each one missing.  The constants of a kernel are fitted
@@ -544,6 +530,49 @@ static double strips_us(const std::vector<int>& strips, const std::vector<int>& 
     const long long rounds = (waves + resident - 1) / resident;
     const int groups = rounds > 1 ? full : std::min(full, (int)((waves + group - 1) / group));
     return row_us * (rows + prologue) * (double)rounds * (1.0 - idle * (full - groups));
+}
+
+// rows per strip of the ensemble's column-marching launch (configuration
+// with bh == 0): whole rounds of resident waves over all members' strips
+static int ens_march_rows(const std::vector<EnsMember>& members, bool fast_arith, double* us = nullptr) {
+    std::vector<int> strips, ny;
+    for (const EnsMember& M : members) {
+        strips.push_back((M.nx + march::kOut - 1) / march::kOut);
+        ny.push_back(M.ny);
+    }
+    // the stages' kernels hold the same number of waves
+    const int resident = resident_waves((const void*)(fast_arith ? ens_march_kernel<true>(march::kStageSecond)
+                                                                 : ens_march_kernel<false>(march::kStageSecond)));
+    const int rows = march_rows(strips.data(), ny.data(), (int)members.size(), resident, 1);
+    if (us) *us = strips_us(strips, ny, rows, resident, 2.65, 2.6, 0.07);
+    return rows;
+}
+
+// Configuration of an ensemble whose caller leaves it open: the marching
+// kernel, or 2-D tiles where a few of them per CU are faster -- 16x16 for
+// members so narrow that strips of 60 columns leave most lanes idle, 32x16 with
+// 512 threads for some launches of three or four a CU.  The estimates (us) are
+// fitted to launches of 16 to 4096 members of 8x8 to 200x133 cells.  us per
+// substep, marching / chosen: 1024 members of 16^2 16.4 / 10.7, 200 of 16x64
+// 15.1 / 9.7, 4096 of 16^2 45.5 / 31.1, 400 of 32^2 15.3 / 14.6; 1024 of 8^2
+// 11.0 marching, 9.7 in 16x16 tiles.
+static int ens_default_config(const std::vector<EnsMember>& members, bool fast_arith) {
+    const int cus = compute_units();
+    auto per_cu = [&](int bw, int bh) {
+        long long tiles = 0;
+        for (const EnsMember& M : members) tiles += (long long)((M.nx + bw - 1) / bw) * ((M.ny + bh - 1) / bh);
+        return (double)((tiles + cus - 1) / cus);
+    };
+    double least;
+    (void)ens_march_rows(members, fast_arith, &least);
+    int cfg = default_tile_config();
+    const double small = per_cu(16, 16), large = per_cu(32, 16);
+    if (small > 2.0 && std::max(6.6 + 0.75 * small, 4.6 + 1.5 * small) < least) {
+        least = std::max(6.6 + 0.75 * small, 4.6 + 1.5 * small);
+        cfg = 3;
+    }
+    if (large > 2.0 && large <= 8.0 && 4.1 + 2.6 * large < least) cfg = 5;
+    return cfg;
 }
 
 static int ens_launch(const gocean_ensemble* E, EnsLaunch L, hipStream_t s) {
@@ -615,7 +644,7 @@ int gocean_ensemble_create(const gocean_member_t* members, int n, int tile_confi
     if (!E) return set_error(GOCEAN_ENOMEM, "host allocation failed");
     E->n = n;
     E->rk_order = members[0].domain.rk_order;
-    E->cfg = tile_config < 0 ? default_tile_config() : tile_config;
+    E->cfg = tile_config;
     E->default_cfg = tile_config < 0;
     bool any_field = false, any_const = false;
     for (int k = 0; k < n; ++k) {
@@ -642,12 +671,9 @@ int gocean_ensemble_create(const gocean_member_t* members, int n, int tile_confi
     for (int k = 0; k < n; ++k)
         E->fits = E->fits && march_fits(members[k].domain.ny, members[k].domain.pitch, members[k].domain.hi_pitch);
     if (E->cfg >= kFirstMarchConfig && !E->fits) {
-        if (tile_config >= 0) {
-            delete E;
-            return set_error(GOCEAN_EINVAL, "tile configuration %d (column marching) needs member planes below 4 GiB",
-                             tile_config);
-        }
-        E->cfg = kDefaultTileConfig;
+        delete E;
+        return set_error(GOCEAN_EINVAL, "tile configuration %d (column marching) needs member planes below 4 GiB",
+                         tile_config);
     }
     E->fast_arith = true;
     E->friction = 0.0f;
@@ -662,13 +688,12 @@ int gocean_ensemble_create(const gocean_member_t* members, int n, int tile_confi
         for (int k = 0; k < n; ++k) { nx[k] = members[k].domain.nx; ny[k] = members[k].domain.ny; }
         E->general = general_tile(E->mode, nx.data(), ny.data(), n);
     }
+    std::vector<EnsMember> shape(n);
+    for (int k = 0; k < n; ++k) { shape[k].nx = members[k].domain.nx; shape[k].ny = members[k].domain.ny; }
+    if (E->default_cfg) E->cfg = E->fits ? ens_default_config(shape, E->fast_arith) : kDefaultTileConfig;
     const TileConfig& tc = (E->mode == kModeZero) ? kTileConfigs[E->cfg] : kGeneralTiles[E->general];
     E->bw = tc.bw; E->bh = tc.bh; E->nt = tc.nt;
-    if (E->bh == 0) {
-        std::vector<EnsMember> shape(n);
-        for (int k = 0; k < n; ++k) { shape[k].nx = members[k].domain.nx; shape[k].ny = members[k].domain.ny; }
-        E->bh = ens_march_rows(shape, E->fast_arith);
-    }
+    if (E->bh == 0) E->bh = ens_march_rows(shape, E->fast_arith);
     std::vector<int> tile_member;
     E->members.resize(n);
     for (int k = 0; k < n; ++k) {
@@ -732,7 +757,7 @@ int gocean_ensemble_set_tile_config(gocean_ensemble_t* E, int tile_config) {
         return set_error(GOCEAN_EINVAL, "tile configuration %d (column marching) needs member planes below 4 GiB",
                          tile_config);
     E->default_cfg = tile_config < 0;
-    if (tile_config < 0) tile_config = E->fits ? default_tile_config() : kDefaultTileConfig;
+    if (tile_config < 0) tile_config = E->fits ? ens_default_config(E->members, E->fast_arith) : kDefaultTileConfig;
     // work already queued may still read the old tables
     if (hipDeviceSynchronize() != hipSuccess) return check_launch("ensemble tile configuration");
     E->cfg = tile_config;
@@ -947,8 +972,8 @@ long long gocean_ensemble_adjoint_setup(gocean_ensemble_t* E, int max_steps) {
     // the faster one; past 24 a CU the strips are.
     const int cus = compute_units();
     const long long per_cu = ((long long)ftiles.size() + cus - 1) / cus;
-    E->rec_march = !(per_cu > 1 && per_cu <= 24 &&
-                     6.5 + 4.0 * (double)per_cu < strips_us(rnx, rny, rbh, rec_resident, 3.9, 2.0, 0.1));
+    E->rec_march = E->fits && !(per_cu > 1 && per_cu <= 24 &&
+                                6.5 + 4.0 * (double)per_cu < strips_us(rnx, rny, rbh, rec_resident, 3.9, 2.0, 0.1));
     for (int k = 0; k < E->n; ++k) {
         EnsMember& M = E->members[k];
         M.astrips_x = snx[k];
@@ -1016,7 +1041,7 @@ struct EnsSegment {
         EnsTapeLaunch L;
         L.members = E->d_members; L.tile_member = E->d_ftile_member;
         L.in = in; L.qn = qn; L.out = out; L.tape = tape; L.Hi = Hi; L.dt = dt; L.rk_step = rk_step;
-        if (E->cfg >= kFirstMarchConfig && E->mode == kModeZero && (E->rec_march || !E->default_cfg)) {
+        if (E->mode == kModeZero && (E->default_cfg ? E->rec_march : E->cfg >= kFirstMarchConfig)) {
             L.tile_member = E->d_rstrip_member;
             const dim3 grid((E->n_rstrips + 3) / 4), block(256);
             if (E->fast_arith) hipLaunchKernelGGL((k_ens_march_tape<true>), grid, block, 0, s, L, E->rec_bh, E->n_rstrips);

@@ -189,10 +189,10 @@ int gocean_adjoint_reverse_kernel(void);
 /* Names of the tile configurations the library is built with; returns the
  * count and writes up to max entries of "BWxBH/threads" into names. */
 int gocean_tile_configs(const char** names, int max);
-/* The configuration a tile_config of -1 selects for an nx x ny domain (or an
- * ensemble whose members average nx*ny cells): the column-marching kernel
- * with balanced rows per strip, whatever the size (planes of 4 GiB or more
- * take a 2-D tile instead). */
+/* The configuration a tile_config of -1 selects for an nx x ny domain: the
+ * column-marching kernel with balanced rows per strip, whatever the size (planes
+ * of 4 GiB or more take a 2-D tile instead).  An ensemble's default is the same,
+ * or a 2-D tile where its members' sizes and number suit that better. */
 int gocean_default_tile_config(int nx, int ny);
 
 /* The constants of the substep kernels' two-instruction division by d (the cell

@@ -3,6 +3,8 @@ a strip of one row on the smallest domains, ragged last strips and rows, and
 more strips than one round of resident waves.  Every configuration gives the
 same bits, so the 2-D tile kernel is the reference."""
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -47,6 +49,30 @@ def test_default_ensemble_equals_tile():
         states.append(ens.state[0].cpu().numpy())
         ens.cleanUp()
     assert H.normal_equal(*states)
+
+
+@pytest.mark.parametrize("n,nx,ny,tile", [(1024, 16, 16, (16, 16)), (200, 16, 64, (16, 16)), (400, 32, 32, (32, 16)),
+                                          (40, 16, 16, None), (300, 60, 16, None)])
+def test_default_ensemble_of_small_members(n, nx, ny, tile):
+    """Many small members take 2-D tiles by default, and give the bits of the
+    marching kernel."""
+    print("default small members", n, nx, ny, flush=True)
+    from SWESimulators import CDKLM16Ensemble, Common, _gocean as G
+    inp, _, _, _ = _case(nx, ny, (1, 2, 1, 2), n, "film")
+    m = dict(nx=nx, ny=ny, dx=inp.dx, dy=inp.dy, f=inp.f, bc=inp.bc, Hi=inp.Hi, eta=inp.eta, hu=inp.hu, hv=inp.hv,
+             wind_x=1e-4)
+    states, tiles = [], []
+    for cfg in (9, None):
+        ens = CDKLM16Ensemble.CDKLM16Ensemble(Common.HIPContext(), [m] * n, dt=0.3, tile_config=cfg)
+        ens.step_n(2)
+        ens.gpu_stream.synchronize()
+        count = ctypes.c_int()
+        G.check(ens.lib.gocean_ensemble_info(ens.handle, None, ctypes.byref(count), None), "info")
+        tiles.append(count.value)
+        states.append(ens.state[0].cpu().numpy())
+        ens.cleanUp()
+    assert H.normal_equal(*states)
+    assert tiles[1] == (tiles[0] if tile is None else n * -(-nx // tile[0]) * -(-ny // tile[1]))
 
 
 @pytest.mark.parametrize("nx,ny", [(2, 2), (61, 5), (300, 1030)])
