@@ -57,7 +57,9 @@ class Simulator(object):
         (Simulator.update_wind_stress, Simulator.py:145-223)."""
         ws = self.wind_stress
         t_max_index = len(ws.t) - 1
-        at = bisect.bisect_left(ws.t, self.t)
+        # in float64: NumPy compares a float32 sample time with a Python float
+        # in float32
+        at = bisect.bisect_left(ws.t, np.float64(self.t))
         t0_index = max(0, at - 1)
         t1_index = min(t_max_index, at)
         new_t0 = ws.t[t0_index]
