@@ -753,7 +753,8 @@ int gocean_ensemble_set_tile_config(gocean_ensemble_t* E, int tile_config) {
     if (!E) return set_error(GOCEAN_EINVAL, "ensemble is NULL");
     if (tile_config >= kNumTileConfigs)
         return set_error(GOCEAN_EINVAL, "tile configuration %d out of range", tile_config);
-    if (tile_config >= kFirstMarchConfig && !E->fits)
+    // rotated and per-cell members march in no configuration
+    if (tile_config >= kFirstMarchConfig && !E->fits && E->mode == kModeZero)
         return set_error(GOCEAN_EINVAL, "tile configuration %d (column marching) needs member planes below 4 GiB",
                          tile_config);
     E->default_cfg = tile_config < 0;

@@ -290,3 +290,30 @@ def test_rk_order_1_ensemble_steps_in_pairs():
     for g, r in zip(ens.download(0), sim.h0):
         assert np.array_equal(g[2:-2, 2:-2], r[2:-2, 2:-2])
     ens.cleanUp()
+
+
+@pytest.mark.parametrize("rotated,accepted", [(True, True), (False, False)])
+def test_marching_configuration_of_planes_past_4_gib(rotated, accepted):
+    """A marching configuration is refused for planes past its 32-bit offsets
+    where it would run; an ensemble of rotated members, which ignores the
+    configuration, accepts it.  No buffers are needed: nothing is launched."""
+    import ctypes
+    from SWESimulators import Common, _gocean as G
+    _say("marching configuration, planes past 4 GiB", rotated)
+    lib = G.load()
+    nx, ny = 65536, 16384
+    m = (G.Member * 1)()
+    m[0].domain = Common.make_domain(nx, ny, 100.0, 100.0, 9.81, 0.0, 1.3, 2, (1, 1, 1, 1), pitch=nx + 4,
+                                     hi_pitch=nx + 5, north_x=0.6 if rotated else 0.0,
+                                     north_y=0.8 if rotated else 1.0)
+    m[0].field_offset = -1
+    h = ctypes.c_void_p()
+    G.check(lib.gocean_ensemble_create(m, 1, -1, ctypes.byref(h)), "ensemble_create")
+    try:
+        rc = lib.gocean_ensemble_set_tile_config(h, 7)
+        assert (rc == 0) == accepted
+        if not accepted:
+            assert "4 GiB" in lib.gocean_last_error().decode()
+        G.check(lib.gocean_ensemble_set_tile_config(h, -1), "default configuration")
+    finally:
+        lib.gocean_ensemble_destroy(h)
