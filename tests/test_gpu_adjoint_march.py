@@ -220,7 +220,7 @@ def test_ensemble_marching_record_equals_tile_record(keep):
                                  f"{H.diff_report(ga, gb, 8)}")
 
 
-@pytest.mark.parametrize("n,size", [(700, (16, 16)), (300, (20, 33)), (40, (20, 12)), (3, (130, 70))])
+@pytest.mark.parametrize("n,size", [(700, (16, 16)), (400, (32, 32)), (40, (20, 12)), (3, (130, 70))])
 def test_default_ensemble_record_follows_the_sizes(n, size):
     """The default configuration records through tiles (the first two) or
     strips of the recording kernel's own height: the same bits as the explicit
@@ -229,7 +229,8 @@ def test_default_ensemble_record_follows_the_sizes(n, size):
     from test_gpu_ensemble import members
     _say("default ensemble record", n, size)
     Common, G, A = _mods()
-    ms = members(seed=11, sizes=(size,) * n)
+    kinds = members(seed=11, sizes=(size,) * 4)
+    ms = [kinds[k % 4] for k in range(n)]
     ref = _ens_run(ms, 1, 3, 3, True, 4)
     for tile in (None, 9):
         got = _ens_run(ms, tile, 3, 3, True, 4)

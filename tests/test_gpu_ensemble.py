@@ -68,6 +68,35 @@ def test_ensemble_matches_oracle(rk_order, tile):
     assert not report, report[:8]
 
 
+@pytest.mark.parametrize("rk_order", [1, 2])
+@pytest.mark.parametrize("tile", [None, 9, 1])
+@pytest.mark.parametrize("rubbed", [(1,), (3,), (0, 2)])
+def test_friction_of_some_members(rk_order, tile, rubbed):
+    """Friction in some members only, the first among them or not: the launch's
+    kernel is chosen by the largest coefficient, and every member keeps its
+    own.  A third of each member is shallow, where friction matters."""
+    from SWESimulators import Common, CDKLM16Ensemble
+    _say("ensemble friction, rk", rk_order, "tile", tile, "members", rubbed)
+    ms = members(seed=21)
+    for k, m in enumerate(ms):
+        m["r"] = 3.0e-3 * (1 + k) if k in rubbed else 0.0
+        w = m["nx"] // 3
+        m["Hi"][:, :w] = 0.3 + 0.1 * m["Hi"][:, :w] / 50.0
+        for q in ("eta", "hu", "hv"):
+            m[q][:, :w] *= 0.01
+    ens = CDKLM16Ensemble.CDKLM16Ensemble(Common.HIPContext(0), ms, rk_order=rk_order, tile_config=tile, dt=0.4)
+    ens.step_n(2)
+    got = [ens.download(k) for k in range(len(ms))]
+    ens.cleanUp()
+    for k, m in enumerate(ms):
+        sim, _ = oracle_member(m, rk_order)
+        sim.step_n(2, np.float32(0.4))
+        for g, r, name in zip(got[k], sim.h0, ("eta", "hu", "hv")):
+            g, r = g[2:-2, 2:-2], r[2:-2, 2:-2]
+            assert H.normal_equal(g, r), (k, name, H.diff_report(g, r))
+
+
+
 def test_graph_replays_match_eager():
     """Replay a captured graph several times with eager work in between;
     every replay must equal the eager result."""

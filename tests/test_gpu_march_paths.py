@@ -113,3 +113,41 @@ def test_march_land_marker_among_the_depths():
     for other in out[1:]:
         for a, b in zip(out[0], other):
             assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("field", ["eta", "hu", "hv", "Hi"])
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf])
+def test_march_non_finite_cells(field, value):
+    """NaN and infinities in single cells, at a strip's inner columns and beside
+    its edges: the marching kernel gives the 2-D tiles' result, NaN in the same
+    cells and the same bits elsewhere, whatever the NaN's sign; cells whose
+    stencil holds none of them are as if there were none, and momentum planted
+    as NaN stays NaN."""
+    print("march non-finite", field, value, flush=True)
+    spots = [(4, 5), (10, 30), (15, 61), (12, 62), (17, 100), (8, 121)]
+    inp, p, Hif, Hm = _case(125, 21, (1, 1, 1, 1), 13, "deep")
+    runs = {}
+    for sign in (1, -1):
+        a = getattr(inp, field).copy()
+        for r, c in spots:
+            a[r, c] = np.copysign(np.float32(value), np.float32(sign)) if np.isnan(value) else value
+        clean, at = getattr(inp, field), {field: a}
+        for tile in (1, 5, MARCH8, MARCH_AUTO, -1):
+            setattr(inp, field, at[field])
+            D = H.DeviceDomain(inp)
+            D.bathymetry_init()
+            h0, h1 = D.state(inp.eta, inp.hu, inp.hv), D.state(inp.eta, inp.hu, inp.hv)
+            D.substep(0.4, 0, h0, h1, tile=tile)
+            runs[sign, tile] = np.stack(D.host(h1))[:, 2:-2, 2:-2]
+            setattr(inp, field, clean)
+    first = runs[1, 1]
+    for key, got in runs.items():
+        assert np.array_equal(first, got, equal_nan=True), key
+    ref = np.stack(O.cdklm_substep(0.4, 0, inp.eta, inp.hu, inp.hv, inp.eta, inp.hu, inp.hv, Hif, Hm, p))[:, 2:-2, 2:-2]
+    far = np.ones(ref.shape[1:], bool)
+    for r, c in spots:
+        far[max(0, r - 2 - 4):r - 2 + 5, max(0, c - 2 - 4):c - 2 + 5] = False
+    assert far.any() and H.normal_equal(first[:, far], ref[:, far])
+    if field in ("hu", "hv") and np.isnan(value):
+        for r, c in spots:
+            assert np.isnan(first[1:, r - 2, c - 2]).any(), (r, c)

@@ -80,8 +80,10 @@ FEATURES = [
 ]
 
 
-# tile configurations: the default 2-D tile and the column-marching strips
-TILES = [-1, 8]
+# tile configurations: the default and fixed column-marching strips, and the
+# 256- and 512-thread 2-D tiles (planes past 4 GiB, ensembles of small members,
+# explicit configurations)
+TILES = [-1, 8, 1, 5]
 
 
 @pytest.mark.parametrize("bcname,bc", BCS)

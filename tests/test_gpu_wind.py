@@ -45,7 +45,7 @@ def _inp(p, Hi, eta, hu, hv):
     return i
 
 
-@pytest.mark.parametrize("tile", [-1, 8])
+@pytest.mark.parametrize("tile", [-1, 8, 1, 5])
 @pytest.mark.parametrize("shape", ["coarse", "same", "thin"])
 @pytest.mark.parametrize("bcname,bc", BCS)
 def test_gridded_wind_substep_bitexact(tile, shape, bcname, bc):
@@ -89,7 +89,7 @@ def _interp(ts, t):
 
 
 @pytest.mark.parametrize("gridded", [False, True])
-@pytest.mark.parametrize("tile", [-1, 8])
+@pytest.mark.parametrize("tile", [-1, 8, 1, 5])
 def test_class_wind_time_series(gridded, tile):
     """CDKLM16.step(30.0) in two calls (12 steps of 2.5 s) over a wind series
     with samples at t = 0, 20 and 60 s: every step takes the bracketing
