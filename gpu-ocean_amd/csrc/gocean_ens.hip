@@ -565,7 +565,7 @@ static int ens_default_config(const std::vector<EnsMember>& members, bool fast_a
     };
     double least;
     (void)ens_march_rows(members, fast_arith, &least);
-    int cfg = default_tile_config();
+    int cfg = kMarchAutoConfig;
     const double small = per_cu(16, 16), large = per_cu(32, 16);
     if (small > 2.0 && std::max(6.6 + 0.75 * small, 4.6 + 1.5 * small) < least) {
         least = std::max(6.6 + 0.75 * small, 4.6 + 1.5 * small);

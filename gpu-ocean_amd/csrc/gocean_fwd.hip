@@ -211,11 +211,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WGRID ? 4 :
 }
 
 int compute_units() {
-    int dev = 0, cus = 256;
+    static std::atomic<int> known{0};
+    int cus = known.load(), dev = 0;
+    if (cus) return cus;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
         (void)hipGetLastError();
-        cus = 256;
+        return 256;
     }
+    known.store(cus);
     return cus;
 }
 
@@ -336,9 +339,7 @@ static void launch_substep_t(SubstepArgs A, hipStream_t s) {
 // 9.3, 1500^2 62.3 / 70.7 / 80.0, 1024 members of 16^2 29.6 / 13.5 / 22.9.
 int general_tile(int mode, const int* nx, const int* ny, int n) {
     constexpr double cost[2][3] = {{1.0, 0.65, 0.65}, {1.0, 0.70, 0.75}};
-    static std::atomic<int> known{0};
-    if (!known.load()) known.store(compute_units());
-    const int cus = known.load();
+    const int cus = compute_units();
     int best = 0;
     double least = 0.0;
     for (int k = 0; k < 3; ++k) {
@@ -409,12 +410,13 @@ static void launch_march_tape(SubstepArgs A, int bh, hipStream_t s) {
 // tile configuration of the recording forward (process-wide; the record is
 // laid out per cell, so every configuration writes the same record); -1: the
 // column-marching kernel (per substep against 32x16/512: 96^2 8.4 / 11.3 us,
-// 512^2 13.7 / 15.1, 1024^2 25.2 / 36.0)
+// 512^2 13.7 / 15.1, 1024^2 25.2 / 36.0), 32x16/512 for a narrow domain
 static int g_record_cfg = -1;
+static bool narrow_domain(int nx, int ny);
 
 int launch_substep_tape(SubstepArgs A, hipStream_t s) {
     int cfg = g_record_cfg;
-    if (cfg < 0) cfg = kMarchAutoConfig;
+    if (cfg < 0) cfg = narrow_domain(A.nx, A.ny) ? 5 : kMarchAutoConfig;
     if (cfg >= kFirstMarchConfig && !march_fits(A.ny, A.pitch, A.hi_pitch)) cfg = 5;
     switch (cfg) {
         case 0: launch_tape_t<32, 8, 256>(A, s); break;
@@ -441,8 +443,12 @@ int substep_mode(const SubstepArgs& A, bool field) {
 // so that they too spread over the chip.  Substep times, marching against the
 // best 2-D tile: 96x80 5.5 / 7.5 us, 512^2 8.5 / 9.1, 1024^2 16.4 / 23.7,
 // 2048^2 43.8 / 74.4; 1024 members of 64^2 78 / 107, 100 of 512^2 270 / 580.
-// The 2-D tile serves rotated grids, per-cell fields and planes of 4 GiB.
-int default_tile_config() { return kMarchAutoConfig; }
+// The 2-D tile serves rotated grids, per-cell fields and planes of 4 GiB, and
+// 16x16 ones (narrow_domain) domains that leave most of a strip's 60 lanes idle
+// and fill the chip all the same: 16x16384 9.9 us against 15.1 marching, with
+// friction 10.2 against 17.4; 16x8193, three tiles a CU, 8.1 against 10.7.
+static bool narrow_domain(int nx, int ny) { return nx <= 16 && (ny + 15) / 16 > 2 * compute_units(); }
+int default_tile_config(int nx, int ny) { return narrow_domain(nx, ny) ? 3 : kMarchAutoConfig; }
 
 // the column-marching kernel addresses a plane with 32-bit byte offsets
 bool march_fits(int ny, int pitch, int hi_pitch) {
@@ -453,7 +459,7 @@ bool march_fits(int ny, int pitch, int hi_pitch) {
 int launch_substep(const SubstepArgs& A, int cfg, bool field, hipStream_t s) {
     const bool fits = march_fits(A.ny, A.pitch, A.hi_pitch);
     if (cfg < 0) {
-        cfg = default_tile_config();
+        cfg = default_tile_config(A.nx, A.ny);
         if (cfg >= kFirstMarchConfig && !fits) cfg = kDefaultTileConfig;
     }
     if (cfg >= kNumTileConfigs)
@@ -740,7 +746,7 @@ int gocean_adjoint_set_record_tile_config(int cfg) {
 
 int gocean_adjoint_record_tile_config(void) { return g_record_cfg; }
 
-int gocean_default_tile_config(int, int) { return default_tile_config(); }
+int gocean_default_tile_config(int nx, int ny) { return default_tile_config(nx, ny); }
 
 int gocean_division_constants(float d, float* high, float* low) {
     clear_error();

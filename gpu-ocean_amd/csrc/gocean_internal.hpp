@@ -26,7 +26,7 @@ int general_tile(int mode, const int* nx, const int* ny, int n);
 // configurations kFirstMarchConfig .. kNumTileConfigs-1 are column marching
 constexpr int kFirstMarchConfig = 7;
 // configuration used when the caller passes -1
-int default_tile_config();
+int default_tile_config(int nx, int ny);
 
 int set_error(int code, const char* fmt, ...);
 void clear_error();

@@ -164,8 +164,8 @@ int gocean_max_dt_static(const gocean_domain_t* d, const float* eta, const float
                          void* stream);
 
 /* Tile configuration (index into gocean_tile_configs; -1, the default: the
- * column-marching kernel) of the
- * recording forward substep the adjoint entry points run
+ * column-marching kernel, or a tile for a long domain at most 16 columns wide)
+ * of the recording forward substep the adjoint entry points run
  * (gocean_adjoint_record / _segment).  Process-wide; every configuration
  * writes the same record.  An ensemble records with its own configuration
  * (gocean_ensemble_set_tile_config): through strips of its recording kernel's
@@ -190,8 +190,8 @@ int gocean_adjoint_reverse_kernel(void);
  * count and writes up to max entries of "BWxBH/threads" into names. */
 int gocean_tile_configs(const char** names, int max);
 /* The configuration a tile_config of -1 selects for an nx x ny domain: the
- * column-marching kernel with balanced rows per strip, whatever the size (planes
- * of 4 GiB or more take a 2-D tile instead).  An ensemble's default is the same,
+ * column-marching kernel with balanced rows per strip, or a 2-D tile for a long
+ * domain at most 16 columns wide (planes of 4 GiB or more take a 2-D tile too).  An ensemble's default is the same,
  * or a 2-D tile where its members' sizes and number suit that better. */
 int gocean_default_tile_config(int nx, int ny);
 

@@ -49,6 +49,16 @@ def test_version_and_configs():
     assert all(b"/" in names[i] for i in range(n))
 
 
+@pytest.mark.parametrize("nx,ny,marching", [(16, 8192, True), (16, 8193, False), (3, 100000, False), (17, 100000, True),
+                                            (512, 512, True), (2, 2, True)])
+def test_default_configuration_of_a_domain(nx, ny, marching):
+    """Marching strips, except for a long domain that fills few of their lanes."""
+    lib = G.load()
+    names = (ctypes.c_char_p * 32)()
+    lib.gocean_tile_configs(names, 32)
+    assert names[lib.gocean_default_tile_config(nx, ny)].startswith(b"march") == marching
+
+
 def _dom(**kw):
     args = dict(nx=32, ny=20, dx=100.0, dy=100.0, g=9.81, r=0.0, theta=1.3, rk_order=2,
                 bc=(1, 1, 1, 1))

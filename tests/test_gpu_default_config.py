@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 TILE = 1
 
 
-@pytest.mark.parametrize("nx,ny", [(2, 3), (61, 5), (96, 80), (503, 301), (1030, 517)])
+@pytest.mark.parametrize("nx,ny", [(2, 3), (61, 5), (96, 80), (503, 301), (1030, 517), (16, 8300), (5, 8193)])
 @pytest.mark.parametrize("bc", [(1, 1, 1, 1), (2, 2, 2, 2), (1, 2, 1, 2)])
 def test_default_equals_tile(nx, ny, bc):
     print("default config", nx, ny, bc, flush=True)
