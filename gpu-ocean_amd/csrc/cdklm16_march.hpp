@@ -35,7 +35,7 @@
 // both.  Hence the wave-uniform fast paths (one compare into a scalar mask
 // decides for the row), constants in vector registers, and rare rows, strips
 // and depths kept in branches of their own.  2048 x 2048, SSP-RK2, 15 rows per
-// strip: 50.9 us per substep before these, 43.8 us after (491 to 400 vector
+// strip: 50.9 us per substep before these, 44.7 us after (491 to 410 vector
 // instructions per cell).
 //
 // Work per output cell: the tile kernel converts (BH+4)(BW+4)-4*4 cells for
@@ -248,7 +248,10 @@ __device__ __forceinline__ Carry slope_fwd(float ec, float er, float ac, float a
 // under the slope's own flip.  `in`: the backward candidates (from the low
 // neighbour); `out`: this cell's forward ones.  ok: every lane of `lanes`
 // has both face depths above face_lo (so no adjustment fired and both
-// faces are wet on this side).
+// faces are wet on this side).  The minimum of the two drops a NaN, but never
+// decides by the other alone: T is NaN with any of the cell's depth and
+// velocity, and then both are (a NaN corner depth makes the cell's velocities
+// NaN).
 // REC: also the slope centre's branch record (tape code byte): the minmod
 // selections of the u and v slopes and of K / L, and which positivity
 // adjustment fired (x: a = u; y: a = v).

@@ -202,7 +202,10 @@ __host__ __device__ __forceinline__ float minmod_raw(float b, float c, float f) 
 
 // The same as a median: the least of three positive candidates, the greatest
 // of three negative ones, zero between them.  Three instructions (min3, max3,
-// med3) against five; the value is minmod_raw's, up to the sign of a zero.
+// med3) against five; the value is minmod_raw's, up to the sign of a zero.  A
+// NaN candidate drops out here, whatever its sign, where minmod_raw drops it
+// from the minimum but takes its sign bit into the agreement; three give zero.
+// Only slopes of cells beside one that is not finite see the difference.
 __device__ __forceinline__ float minmod3(float b, float c, float f) {
     return __builtin_amdgcn_fmed3f(fminf(fminf(b, c), f), fmaxf(fmaxf(b, c), f), 0.0f);
 }

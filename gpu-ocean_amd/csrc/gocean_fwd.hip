@@ -237,10 +237,13 @@ int resident_waves(const void* kernel) {
 // Rows per strip for a column-marching kernel over domains of the given
 // strip counts and heights: each wave's time grows with its rows plus about
 // three rows of prologue, and waves run in rounds of `resident`; pick the
-// row count (least..256) with the least rounds * (rows + 3).  Measured over
-// fixed row counts, the choice is the best or within 3 % of it from 96x80 (1
-// row) over 512^2 (1), 1024^2 (4) and 2048^2 (15) to 1024 members of 64^2 and
-// 100 of 512^2.
+// row count (least..256) with the least rounds * (rows + 3).  us per substep of
+// the choice, of 8 and of 16 rows: 96x80 5.7 / 13.7 / 22.9, 512^2 8.9 / 14.0 /
+// 23.1, 1024^2 16.6 / 19.2 / 26.9, 1500^2 26.9 / 26.7 / 33.0, 2048^2 (15 rows)
+// 44.7 / 45.0 / 46.6, 4096^2 170 / 179 / 171.  Under the profiler 8 rows at
+// 2048^2 are 4 % faster than 15 (47.5 and 49.4).  Only the latency of the waves
+// is counted: where two row counts are level, the lower one, which does more
+// work in prologues, is taken.
 int march_rows(const int* strips, const int* ny, int n, int resident, int least) {
     int best = least;
     double best_cost = 1e300;
@@ -441,8 +444,8 @@ int substep_mode(const SubstepArgs& A, bool field) {
 // Default configuration: the column-marching kernel with balanced rows per
 // strip, for every size.  Small domains get strips of few rows (march_rows),
 // so that they too spread over the chip.  Substep times, marching against the
-// best 2-D tile: 96x80 5.5 / 7.5 us, 512^2 8.5 / 9.1, 1024^2 16.4 / 23.7,
-// 2048^2 43.8 / 74.4; 1024 members of 64^2 78 / 107, 100 of 512^2 270 / 580.
+// best 2-D tile: 96x80 5.5 / 7.5 us, 512^2 8.9 / 9.1, 1024^2 16.4 / 23.7,
+// 2048^2 44.7 / 74.4; 1024 members of 64^2 75 / 82, 100 of 512^2 256 / 580.
 // The 2-D tile serves rotated grids, per-cell fields and planes of 4 GiB, and
 // 16x16 ones (narrow_domain) domains that leave most of a strip's 60 lanes idle
 // and fill the chip all the same: 16x16384 9.9 us against 15.1 marching, with
