@@ -554,9 +554,10 @@ static int ens_march_rows(const std::vector<EnsMember>& members, bool fast_arith
 // 512 threads for some launches of three or four a CU.  The estimates (us) are
 // fitted to launches of 16 to 4096 members of 8x8 to 200x133 cells.  us per
 // substep, marching / chosen: 1024 members of 16^2 16.4 / 10.7, 200 of 16x64
-// 15.1 / 9.7, 4096 of 16^2 45.5 / 31.1, 400 of 32^2 15.3 / 14.6; 1024 of 8^2
-// 11.0 marching, 9.7 in 16x16 tiles.
-static int ens_default_config(const std::vector<EnsMember>& members, bool fast_arith) {
+// 15.1 / 9.7, 4096 of 16^2 45.5 / 31.1, 400 of 32^2 15.3 / 14.6, 1024 of 8^2
+// 11.0 / 9.7.
+// rows: those of the marching launch.
+static int ens_default_config(const std::vector<EnsMember>& members, bool fast_arith, int* rows) {
     const int cus = compute_units();
     auto per_cu = [&](int bw, int bh) {
         long long tiles = 0;
@@ -564,7 +565,7 @@ static int ens_default_config(const std::vector<EnsMember>& members, bool fast_a
         return (double)((tiles + cus - 1) / cus);
     };
     double least;
-    (void)ens_march_rows(members, fast_arith, &least);
+    *rows = ens_march_rows(members, fast_arith, &least);
     int cfg = kMarchAutoConfig;
     const double small = per_cu(16, 16), large = per_cu(32, 16);
     if (small > 2.0 && std::max(6.6 + 0.75 * small, 4.6 + 1.5 * small) < least) {
@@ -677,10 +678,11 @@ int gocean_ensemble_create(const gocean_member_t* members, int n, int tile_confi
     }
     E->fast_arith = true;
     E->friction = 0.0f;
+    std::vector<SubstepDerived> derived(n);
     for (int k = 0; k < n; ++k) {
         const gocean_domain_t& d = members[k].domain;
-        SubstepDerived D;
-        E->fast_arith = fast_arith(d.g, d.dx, d.dy, d.depth_cutoff, D) && E->fast_arith;
+        derived[k] = substep_derive(d.dx, d.dy, d.g, d.theta, d.f, d.flux_slope_eps, d.depth_cutoff, d.land_value);
+        E->fast_arith = fast_arith(d.g, d.dx, d.dy, d.depth_cutoff, derived[k]) && E->fast_arith;
         E->friction = std::max(E->friction, d.r);
     }
     if (E->mode != kModeZero) {
@@ -690,10 +692,12 @@ int gocean_ensemble_create(const gocean_member_t* members, int n, int tile_confi
     }
     std::vector<EnsMember> shape(n);
     for (int k = 0; k < n; ++k) { shape[k].nx = members[k].domain.nx; shape[k].ny = members[k].domain.ny; }
-    if (E->default_cfg) E->cfg = E->fits ? ens_default_config(shape, E->fast_arith) : kDefaultTileConfig;
+    int rows = 0;
+    if (E->default_cfg)
+        E->cfg = E->fits && E->mode == kModeZero ? ens_default_config(shape, E->fast_arith, &rows) : kDefaultTileConfig;
     const TileConfig& tc = (E->mode == kModeZero) ? kTileConfigs[E->cfg] : kGeneralTiles[E->general];
     E->bw = tc.bw; E->bh = tc.bh; E->nt = tc.nt;
-    if (E->bh == 0) E->bh = ens_march_rows(shape, E->fast_arith);
+    if (E->bh == 0) E->bh = rows ? rows : ens_march_rows(shape, E->fast_arith);
     std::vector<int> tile_member;
     E->members.resize(n);
     for (int k = 0; k < n; ++k) {
@@ -718,9 +722,7 @@ int gocean_ensemble_create(const gocean_member_t* members, int n, int tile_confi
         M.wind_x = wind_lerp(m.wind.t, m.wind.x0, m.wind.x1);
         M.wind_y = wind_lerp(m.wind.t, m.wind.y0, m.wind.y1);
         M.bc_n = d.bc_north; M.bc_e = d.bc_east; M.bc_s = d.bc_south; M.bc_w = d.bc_west;
-        static_cast<SubstepDerived&>(M) =
-            substep_derive(d.dx, d.dy, d.g, d.theta, d.f, d.flux_slope_eps, d.depth_cutoff, d.land_value);
-        (void)fast_arith(d.g, d.dx, d.dy, d.depth_cutoff, M);
+        static_cast<SubstepDerived&>(M) = derived[k];
         if (m.state_offset < 0 || m.hi_offset < 0 || m.hm_offset < 0) {
             delete E;
             return set_error(GOCEAN_EINVAL, "member %d: negative buffer offset", k);
@@ -758,13 +760,16 @@ int gocean_ensemble_set_tile_config(gocean_ensemble_t* E, int tile_config) {
         return set_error(GOCEAN_EINVAL, "tile configuration %d (column marching) needs member planes below 4 GiB",
                          tile_config);
     E->default_cfg = tile_config < 0;
-    if (tile_config < 0) tile_config = E->fits ? ens_default_config(E->members, E->fast_arith) : kDefaultTileConfig;
+    int rows = 0;
+    if (tile_config < 0)
+        tile_config = E->fits && E->mode == kModeZero ? ens_default_config(E->members, E->fast_arith, &rows)
+                                                      : kDefaultTileConfig;
     // work already queued may still read the old tables
     if (hipDeviceSynchronize() != hipSuccess) return check_launch("ensemble tile configuration");
     E->cfg = tile_config;
     const TileConfig& tc = (E->mode == kModeZero) ? kTileConfigs[E->cfg] : kGeneralTiles[E->general];
     E->bw = tc.bw; E->bh = tc.bh; E->nt = tc.nt;
-    if (E->bh == 0) E->bh = ens_march_rows(E->members, E->fast_arith);
+    if (E->bh == 0) E->bh = rows ? rows : ens_march_rows(E->members, E->fast_arith);
     std::vector<int> tile_member;
     for (int k = 0; k < E->n; ++k) {
         EnsMember& M = E->members[k];
