@@ -130,6 +130,13 @@ __device__ __forceinline__ float flag_land(float h, const Consts& K) {
 // turn the condition into a vector of 0 / 1, two more vector instructions)
 __device__ __forceinline__ bool none(bool c) { return __builtin_amdgcn_ballot_w64(c) == 0ull; }
 
+// every lane of `lanes` has a and b above c, and neither is NaN: two compares
+// and a scalar or (a compare of fminf(a, b), as many vector instructions, would
+// drop a NaN -- the face depth of a dry cell with an infinite corner is one)
+__device__ __forceinline__ bool both_above(float a, float b, float c, unsigned long long lanes) {
+    return ((__builtin_amdgcn_ballot_w64(!(a > c)) | __builtin_amdgcn_ballot_w64(!(b > c))) & lanes) == 0ull;
+}
+
 // marks code that few rows or strips run: the empty volatile asm keeps the
 // compiler from executing it unconditionally behind selects
 __device__ __forceinline__ void rare() { asm volatile(""); }
@@ -248,10 +255,7 @@ __device__ __forceinline__ Carry slope_fwd(float ec, float er, float ac, float a
 // under the slope's own flip.  `in`: the backward candidates (from the low
 // neighbour); `out`: this cell's forward ones.  ok: every lane of `lanes`
 // has both face depths above face_lo (so no adjustment fired and both
-// faces are wet on this side).  The minimum of the two drops a NaN, but never
-// decides by the other alone: T is NaN with any of the cell's depth and
-// velocity, and then both are (a NaN corner depth makes the cell's velocities
-// NaN).
+// faces are wet on this side).
 // REC: also the slope centre's branch record (tape code byte): the minmod
 // selections of the u and v slopes and of K / L, and which positivity
 // adjustment fired (x: a = u; y: a = v).
@@ -281,7 +285,7 @@ __device__ __forceinline__ void slope_rest(float el, float ec, float er, float a
         const uint32_t ad = !(dhi > 0.0f) ? 2u : (!(dlo > 0.0f) ? 1u : 0u);
         *code8 = (SGN < 0 ? (sa | (sb << 2)) : (sb | (sa << 2))) | (sk << 4) | (ad << 6);
     }
-    ok = (__builtin_amdgcn_ballot_w64(!(fminf(dlo, dhi) > K.face_lo)) & lanes) == 0ull;
+    ok = both_above(dlo, dhi, K.face_lo, lanes);
     if (!ok || fix) {
         rare();
         bool adj = false;
@@ -299,7 +303,7 @@ __device__ __forceinline__ void slope_rest(float el, float ec, float er, float a
             dlo = elo - T;
             dhi = ehi + T;
         }
-        ok = (__builtin_amdgcn_ballot_w64(!(fminf(dlo, dhi) > K.face_lo)) & lanes) == 0ull;
+        ok = both_above(dlo, dhi, K.face_lo, lanes);
     }
 }
 

@@ -115,17 +115,22 @@ def test_march_land_marker_among_the_depths():
             assert np.array_equal(a, b)
 
 
+SINGLE = [(4, 5), (10, 30), (15, 61), (12, 62), (17, 100), (8, 121)]
+PAIRS = [(4, 5), (4, 6), (8, 20), (8, 22), (14, 40), (16, 40), (12, 60), (12, 62), (9, 100), (10, 100), (19, 121), (21, 121)]
+
+
 @pytest.mark.parametrize("field", ["eta", "hu", "hv", "Hi"])
 @pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf])
-def test_march_non_finite_cells(field, value):
-    """NaN and infinities in single cells, at a strip's inner columns and beside
-    its edges: the marching kernel gives the 2-D tiles' result, NaN in the same
-    cells and the same bits elsewhere, whatever the NaN's sign; cells whose
-    stencil holds none of them are as if there were none, and momentum planted
-    as NaN stays NaN."""
+@pytest.mark.parametrize("spots", [SINGLE, PAIRS], ids=["single", "pairs"])
+def test_march_non_finite_cells(field, value, spots):
+    """NaN and infinities in
+    single cells and in cells one or two apart in x or y, at a strip's inner
+    columns and beside its edges: the marching kernel gives the 2-D tiles'
+    result, NaN in the same cells and the same bits elsewhere, whatever the
+    NaN's sign; cells whose stencil holds none of them are as if there were
+    none, and momentum planted as NaN stays NaN."""
     print("march non-finite", field, value, flush=True)
-    spots = [(4, 5), (10, 30), (15, 61), (12, 62), (17, 100), (8, 121)]
-    inp, p, Hif, Hm = _case(125, 21, (1, 1, 1, 1), 13, "deep")
+    inp, p, Hif, Hm = _case(125, 21, (1, 1, 1, 1), 13, "deep", dx=100.0)
     runs = {}
     for sign in (1, -1):
         a = getattr(inp, field).copy()
