@@ -137,6 +137,8 @@ __device__ __forceinline__ bool both_above(float a, float b, float c, unsigned l
     return ((__builtin_amdgcn_ballot_w64(!(a > c)) | __builtin_amdgcn_ballot_w64(!(b > c))) & lanes) == 0ull;
 }
 
+__device__ __forceinline__ bool is_inf(float v) { return fabsf(v) == INFINITY; }
+
 // marks code that few rows or strips run: the empty volatile asm keeps the
 // compiler from executing it unconditionally behind selects
 __device__ __forceinline__ void rare() { asm volatile(""); }
@@ -279,6 +281,7 @@ __device__ __forceinline__ void slope_rest(float el, float ec, float er, float a
     dlo = elo - T;
     dhi = ehi + T;
     if constexpr (REC) {
+        if (FAST && is_inf(T)) T = dlo = dhi = NAN;
         const uint32_t sa = minmod_sel(in.a, ca, out.a);
         const uint32_t sb = minmod_sel(in.b, cb, out.b);
         const uint32_t sk = minmod_sel(in.K, ce, out.K);
@@ -288,6 +291,9 @@ __device__ __forceinline__ void slope_rest(float el, float ec, float er, float a
     ok = both_above(dlo, dhi, K.face_lo, lanes);
     if (!ok || fix) {
         rare();
+        // past 1e37 the numerators overflow; an infinite T (one of the depths
+        // is then -inf or NaN, so the row comes here) is NaN as in div_r
+        if (FAST && is_inf(T)) T = dlo = dhi = NAN;
         bool adj = false;
         const bool alo = !(dlo > 0.0f), ahi = !(dhi > 0.0f);
         if constexpr (SGN < 0) {
@@ -300,6 +306,7 @@ __device__ __forceinline__ void slope_rest(float el, float ec, float er, float a
         if (adj || lane_fix) {
             T = (SGN < 0) ? div_k<FAST>(Kv + db, K.two_g, K.r_two_g, K.l_two_g)
                           : div_k<FAST>(Kv - db, K.two_g, K.r_two_g, K.l_two_g);
+            if (FAST && is_inf(T)) T = NAN;
             dlo = elo - T;
             dhi = ehi + T;
         }

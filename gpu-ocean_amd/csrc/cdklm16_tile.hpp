@@ -287,7 +287,8 @@ __device__ __forceinline__ float div_r(float n, float d, float r) {
 // host chooses l and enables the form (SubstepArgs fast_arith()) only for
 // divisors for which it has checked every float significand of n (divisor_low
 // in gocean_fwd.hip); otherwise div_r runs.  Quotients below 2^-126 r / |l|,
-// where n l is subnormal, can be one unit in the last place off.
+// where n l is subnormal, can be one unit in the last place off.  An infinite
+// quotient is infinite or NaN by the sign of l, where div_r gives NaN.
 template <bool FAST>
 __device__ __forceinline__ float div_k(float n, float d, float r, float l) {
     if constexpr (FAST) return fmaf(n, r, n * l);

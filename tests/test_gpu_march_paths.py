@@ -119,11 +119,14 @@ SINGLE = [(4, 5), (10, 30), (15, 61), (12, 62), (17, 100), (8, 121)]
 PAIRS = [(4, 5), (4, 6), (8, 20), (8, 22), (14, 40), (16, 40), (12, 60), (12, 62), (9, 100), (10, 100), (19, 121), (21, 121)]
 
 
-@pytest.mark.parametrize("field", ["eta", "hu", "hv", "Hi"])
-@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf])
+MAX = float(np.finfo(np.float32).max)
+
+
+@pytest.mark.parametrize("field,value", [(f, v) for f in ("eta", "hu", "hv", "Hi") for v in (np.nan, np.inf, -np.inf)]
+                         + [("Hi", v) for v in (MAX, -MAX, 9.96921e36, -9.96921e36)])
 @pytest.mark.parametrize("spots", [SINGLE, PAIRS], ids=["single", "pairs"])
 def test_march_non_finite_cells(field, value, spots):
-    """NaN and infinities in
+    """NaN and infinities, and the values files mark missing depths with, in
     single cells and in cells one or two apart in x or y, at a strip's inner
     columns and beside its edges: the marching kernel gives the 2-D tiles'
     result, NaN in the same cells and the same bits elsewhere, whatever the
